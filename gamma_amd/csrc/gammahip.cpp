@@ -2076,111 +2076,179 @@ GH_HD void body_c2p_batch(long long s, const double* st, const double* guess, co
 namespace {
 using namespace gh::mlp;
 
-// normalised features and targets of raw states (D, |S|, tau, p)
+// normalised features and target of raw states (D, |S|, tau, p), one float4 a state
 __global__ void k_mlp_prepare(const float* __restrict__ w, const double* __restrict__ st, long long n,
-                              float* __restrict__ X, float* __restrict__ T) {
+                              float4* __restrict__ XT) {
   long long s = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= n) return;
   double D = st[4 * s], S = st[4 * s + 1], tau = st[4 * s + 2], p = st[4 * s + 3];
-  features(w, D, S, tau, X + 3 * s);
+  float x[3];
+  features(w, D, S, tau, x);
   double lpd = log(p / (D > 1e-300 ? D : 1e-300));
-  T[s] = (float)((lpd - w[ONORM + 6]) * w[ONORM + 7]);
+  XT[s] = make_float4(x[0], x[1], x[2], (float)((lpd - w[ONORM + 6]) * w[ONORM + 7]));
 }
 
-// gradient of the mean squared error over the samples idx[0..nb) (FP32
-// forward/backward, one wavefront of 64 samples per block), accumulated into g
-__global__ void __launch_bounds__(64) k_mlp_grad(const float* __restrict__ w, const float* __restrict__ X,
-                                                 const float* __restrict__ T, const long long* __restrict__ idx,
-                                                 int nb, float* __restrict__ g, float* __restrict__ loss) {
-  __shared__ float h1s[64][H + 1], zs[64][H + 1], dys[64], xs[64][3];
-  int t = threadIdx.x;
-  int s = blockIdx.x * 64 + t;
-  bool valid = s < nb;
-  float x[3] = {0.f, 0.f, 0.f}, h1[H], h2[H], dy = 0.f;
-  if (valid) {
-    long long k = idx[s];
-    x[0] = X[3 * k]; x[1] = X[3 * k + 1]; x[2] = X[3 * k + 2];
-    float y = forward_f32(w, x, h1, h2);
-    float e = y - T[k];
-    dy = 2.f * e / nb;
-    atomicAdd(loss, e * e / nb);
-  } else {
-    for (int o = 0; o < H; ++o) { h1[o] = 0.f; h2[o] = 0.f; }
-  }
-  for (int o = 0; o < H; ++o) { h1s[t][o] = h1[o]; zs[t][o] = h2[o]; }
-  dys[t] = dy;
-  xs[t][0] = x[0]; xs[t][1] = x[1]; xs[t][2] = x[2];
-  __syncthreads();
-  {   // output layer: dw3[c], db3
-    float a = 0.f;
-    for (int q = 0; q < 64; ++q) a += dys[q] * zs[q][t];
-    atomicAdd(&g[OW3 + t], a);
-    if (t == 0) {
-      float b = 0.f;
-      for (int q = 0; q < 64; ++q) b += dys[q];
-      atomicAdd(&g[OB3], b);
-    }
-  }
-  __syncthreads();
-  for (int o = 0; o < H; ++o) zs[t][o] = zs[t][o] > 0.f ? dys[t] * w[OW3 + o] : 0.f;   // dz2
-  __syncthreads();
-  {   // hidden layer: dW2[o=t][i], db2[t]
-    float b = 0.f;
-    for (int q = 0; q < 64; ++q) b += zs[q][t];
-    atomicAdd(&g[OB2 + t], b);
-    for (int i = 0; i < H; ++i) {
-      float a = 0.f;
-      for (int q = 0; q < 64; ++q) a += zs[q][t] * h1s[q][i];
-      atomicAdd(&g[OW2 + t * H + i], a);
-    }
-  }
-  __syncthreads();
-  {   // dz1 of this sample (row t), then dW1, db1
-    float dz1[H];
-    for (int i = 0; i < H; ++i) {
-      float a = 0.f;
-      for (int o = 0; o < H; ++o) a += w[OW2 + o * H + i] * zs[t][o];
-      dz1[i] = h1s[t][i] > 0.f ? a : 0.f;
-    }
-    __syncthreads();
-    for (int i = 0; i < H; ++i) h1s[t][i] = dz1[i];
-  }
-  __syncthreads();
-  {
-    float b = 0.f, a0 = 0.f, a1 = 0.f, a2 = 0.f;
-    for (int q = 0; q < 64; ++q) {
-      float z = h1s[q][t];
-      b += z; a0 += z * xs[q][0]; a1 += z * xs[q][1]; a2 += z * xs[q][2];
-    }
-    atomicAdd(&g[OB1 + t], b);
-    atomicAdd(&g[OW1 + t * 3], a0);
-    atomicAdd(&g[OW1 + t * 3 + 1], a1);
-    atomicAdd(&g[OW1 + t * 3 + 2], a2);
-  }
-}
-
-// Adam (Kingma & Ba 2015) on the trained entries; clears the gradient
-__global__ void k_mlp_adam(float* w, float* g, float* m, float* v, int step, float lr) {
-  int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= NTRAIN) return;
-  const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-  float gg = g[k];
-  m[k] = b1 * m[k] + (1.f - b1) * gg;
-  v[k] = b2 * v[k] + (1.f - b2) * gg * gg;
-  float mh = m[k] / (1.f - powf(b1, (float)step)), vh = v[k] / (1.f - powf(b2, (float)step));
-  w[k] -= lr * mh / (sqrtf(vh) + eps);
-  g[k] = 0.f;
-}
-
-// minibatch indices drawn with replacement (SplitMix64 counter stream)
-__global__ void k_mlp_sample(long long* idx, int nb, long long n, unsigned long long seed, long long step) {
-  int s = blockIdx.x * blockDim.x + threadIdx.x;
+// state s of minibatch `step`, drawn with replacement (SplitMix64 counter stream)
+__device__ void mlp_draw(const float4* __restrict__ XT, float4* __restrict__ xb, int s, int nb, long long n,
+                         unsigned long long seed, long long step) {
   if (s >= nb) return;
   unsigned long long z = seed + (unsigned long long)(step * (long long)nb + s + 1) * 0x9E3779B97F4A7C15ull;
   z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
   z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
   z ^= z >> 31;
-  idx[s] = (long long)(z % (unsigned long long)n);
+  xb[s] = XT[z % (unsigned long long)n];
+}
+__global__ void k_mlp_draw(const float4* __restrict__ XT, float4* __restrict__ xb, int nb, long long n,
+                           unsigned long long seed, long long step) {
+  mlp_draw(XT, xb, (int)(blockIdx.x * blockDim.x + threadIdx.x), nb, n, seed, step);
+}
+
+// Gradient of the mean squared error over the states xb[0..nb), FP32 forward
+// and backward: workgroup b sums tiles b, b + gridDim, ... of TS states into
+// its own row of `part` (NTRAIN entries, then the loss), which k_mlp_adam sums.
+// The three 64-wide products of a tile (hidden layer, its weight gradient, the
+// first layer's error) run as v_mfma_f32_16x16x4_f32 with FP32 accumulation,
+// wavefront v on columns (rows of the weight gradient) 16 v .. 16 v + 15;
+// everything else of a column stays in the lanes that hold it.
+// The pass is bound by latency (0.1 GFLOP a step): 32 states a tile put 128
+// workgroups on a batch of 4096, and rows stored side by side replace
+// 4481 atomic sums per workgroup at a stride of one line each, which took
+// 90 of the pass's 105 us.
+constexpr int TS = 32;                 // states per tile
+constexpr int TLD = H + 4;             // LDS row stride: 16 rows x 4 columns fall on 64 banks
+constexpr int TMAX = 256;              // most workgroups (rows of partial sums)
+constexpr int GROW = (NTRAIN + 1 + 63) / 64 * 64;
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+__global__ void __launch_bounds__(256) k_mlp_grad(const float* __restrict__ w, const float4* __restrict__ xb,
+                                                  int nb, float* __restrict__ part) {
+  __shared__ __align__(16) float W2[H * TLD], H1[TS * TLD], Z2[TS * TLD];
+  __shared__ float4 xs[TS];
+  __shared__ float yp[4][TS], dys[TS];
+  int t = (int)threadIdx.x, wv = t >> 6, l = t & 63, c = l & 15, g = l >> 4, col = 16 * wv + c;
+  for (int e = t; e < H * H / 4; e += 256)
+    *(float4*)&W2[(e >> 4) * TLD + 4 * (e & 15)] = ((const float4*)(w + OW2))[e];
+  float b2 = w[OB2 + col], w3 = w[OW3 + col];
+  float b1 = w[OB1 + l], w10 = w[OW1 + 3 * l], w11 = w[OW1 + 3 * l + 1], w12 = w[OW1 + 3 * l + 2];
+  floatx4 gw2[4] = {floatx4{}, floatx4{}, floatx4{}, floatx4{}};
+  float gw3 = 0.f, gb2 = 0.f, gb1 = 0.f, gw1[3] = {0.f, 0.f, 0.f}, gb3 = 0.f, loss = 0.f;
+  int ntile = (nb + TS - 1) / TS;
+  for (int tile = (int)blockIdx.x; tile < ntile; tile += (int)gridDim.x) {
+    __syncthreads();
+    if (t < TS) xs[t] = tile * TS + t < nb ? xb[tile * TS + t] : make_float4(0.f, 0.f, 0.f, 0.f);
+    __syncthreads();
+    for (int q = 0; q < TS / 4; ++q) {                       // layer 1
+      float4 x = xs[wv * (TS / 4) + q];
+      float a = b1 + w10 * x.x + w11 * x.y + w12 * x.z;
+      H1[(wv * (TS / 4) + q) * TLD + l] = a > 0.f ? a : 0.f;
+    }
+    __syncthreads();
+    floatx4 z[2] = {floatx4{}, floatx4{}};                   // layer 2: rows 16 m + 4 g + r, column col
+#pragma unroll
+    for (int kk = 0; kk < H / 4; ++kk) {
+      int k = 4 * kk + g;
+      float b = W2[col * TLD + k];
+      for (int m = 0; m < 2; ++m)
+        z[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(H1[(16 * m + c) * TLD + k], b, z[m], 0, 0, 0);
+    }
+    for (int m = 0; m < 2; ++m)
+      for (int r = 0; r < 4; ++r) {
+        float v = z[m][r] + b2;
+        z[m][r] = v > 0.f ? v : 0.f;
+        float y = w3 * z[m][r];
+        for (int o = 1; o < 16; o <<= 1) y += __shfl_xor(y, o, 64);
+        if (c == 0) yp[wv][16 * m + 4 * g + r] = y;
+      }
+    __syncthreads();
+    if (t < TS) {
+      float y = w[OB3] + ((yp[0][t] + yp[1][t]) + (yp[2][t] + yp[3][t]));
+      float e = tile * TS + t < nb ? y - xs[t].w : 0.f, dy = 2.f * e / nb;
+      dys[t] = dy;
+      gb3 += dy;
+      loss += e * e / nb;
+    }
+    __syncthreads();
+    for (int m = 0; m < 2; ++m)
+      for (int r = 0; r < 4; ++r) {
+        int row = 16 * m + 4 * g + r;
+        float dy = dys[row], z2 = z[m][r] > 0.f ? dy * w3 : 0.f;
+        gw3 += dy * z[m][r];
+        gb2 += z2;
+        Z2[row * TLD + col] = z2;
+      }
+    __syncthreads();
+#pragma unroll
+    for (int kk = 0; kk < TS / 4; ++kk) {                    // dW2: rows 16 wv + 4 g + r, columns 16 q + c
+      int s = 4 * kk + g;
+      float a = Z2[s * TLD + col];
+      for (int q = 0; q < 4; ++q)
+        gw2[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, H1[s * TLD + 16 * q + c], gw2[q], 0, 0, 0);
+    }
+    floatx4 d[2] = {floatx4{}, floatx4{}};                   // dH1
+#pragma unroll
+    for (int kk = 0; kk < H / 4; ++kk) {
+      int o = 4 * kk + g;
+      float b = W2[o * TLD + col];
+      for (int m = 0; m < 2; ++m)
+        d[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(Z2[(16 * m + c) * TLD + o], b, d[m], 0, 0, 0);
+    }
+    for (int m = 0; m < 2; ++m)
+      for (int r = 0; r < 4; ++r) {
+        int row = 16 * m + 4 * g + r;
+        float z1 = H1[row * TLD + col] > 0.f ? d[m][r] : 0.f;
+        float4 x = xs[row];
+        gb1 += z1; gw1[0] += z1 * x.x; gw1[1] += z1 * x.y; gw1[2] += z1 * x.z;
+      }
+  }
+  float* P = part + (long long)blockIdx.x * GROW;
+  for (int q = 0; q < 4; ++q)
+    for (int r = 0; r < 4; ++r) P[OW2 + (16 * wv + 4 * g + r) * H + 16 * q + c] = gw2[q][r];
+  for (int o = 16; o < 64; o <<= 1) {
+    gw3 += __shfl_xor(gw3, o, 64); gb2 += __shfl_xor(gb2, o, 64); gb1 += __shfl_xor(gb1, o, 64);
+    for (int k = 0; k < 3; ++k) gw1[k] += __shfl_xor(gw1[k], o, 64);
+  }
+  if (g == 0) {
+    P[OW3 + col] = gw3; P[OB2 + col] = gb2; P[OB1 + col] = gb1;
+    for (int k = 0; k < 3; ++k) P[OW1 + 3 * col + k] = gw1[k];
+  }
+  if (wv == 0) {
+    for (int o = 1; o < TS; o <<= 1) { gb3 += __shfl_xor(gb3, o, 64); loss += __shfl_xor(loss, o, 64); }
+    if (t == 0) { P[OB3] = gb3; P[NTRAIN] = loss; }
+  }
+}
+
+// Sums the workgroups' gradients (four threads an entry), then either stores
+// the sums (gout: the gradient entry point) or takes an Adam step (Kingma & Ba
+// 2015) with bias corrections c1 = 1 - b1^step, c2 = 1 - b2^step; the loss goes
+// to *loss.  In training the workgroups past the parameters gather the next
+// step's minibatch meanwhile, which depends on no weight.
+constexpr int ADAM_WG = GROW / 64;
+__global__ void __launch_bounds__(256) k_mlp_adam(const float* __restrict__ part, int rows, float* __restrict__ w,
+                                                  float* __restrict__ m, float* __restrict__ v, float c1, float c2,
+                                                  float lr, float* __restrict__ gout, float* __restrict__ loss,
+                                                  const float4* __restrict__ XT, float4* __restrict__ xb, int nb,
+                                                  long long n, unsigned long long seed, long long step) {
+  if ((int)blockIdx.x >= ADAM_WG) {
+    mlp_draw(XT, xb, ((int)blockIdx.x - ADAM_WG) * 256 + (int)threadIdx.x, nb, n, seed, step);
+    return;
+  }
+  __shared__ float sm[4][64];
+  int t = (int)threadIdx.x, k = (int)blockIdx.x * 64 + (t & 63);
+  float gg = 0.f;
+  if (k <= NTRAIN) {
+#pragma unroll 8
+    for (int b = t >> 6; b < rows; b += 4) gg += part[(long long)b * GROW + k];
+  }
+  sm[t >> 6][t & 63] = gg;
+  __syncthreads();
+  if (t >= 64 || k > NTRAIN) return;
+  gg = (sm[0][t] + sm[1][t]) + (sm[2][t] + sm[3][t]);
+  if (k == NTRAIN) { *loss = gg; return; }
+  if (gout) { gout[k] = gg; return; }
+  const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+  float mk = b1 * m[k] + (1.f - b1) * gg, vk = b2 * v[k] + (1.f - b2) * gg * gg;
+  m[k] = mk;
+  v[k] = vk;
+  w[k] -= lr * (mk / c1) / (sqrtf(vk / c2) + eps);
 }
 
 // batch inference: pressure guesses of raw states; mfma = 1 runs the BF16 MFMA
@@ -3529,23 +3597,26 @@ int gammahip_mlp_train(const double* states, long long n, float* params, int ste
   if (n < 1 || batch < 64 || steps < 1) return plain_fail("bad training arguments");
   DevBuf B;
   double* st = B.get<double>(4 * n);
-  float *w = B.get<float>(NPARAM), *g = B.get<float>(NPARAM), *m = B.get<float>(NPARAM), *v = B.get<float>(NPARAM);
-  float *X = B.get<float>(3 * n), *T = B.get<float>(n), *loss = B.get<float>(1);
-  long long* idx = B.get<long long>(batch);
-  if (!st || !w || !g || !m || !v || !X || !T || !loss || !idx) return plain_fail("allocation failed");
+  float *w = B.get<float>(NPARAM), *m = B.get<float>(NPARAM), *v = B.get<float>(NPARAM);
+  float4 *XT = B.get<float4>(n), *xb = B.get<float4>(batch);
+  int rows = std::min((batch + TS - 1) / TS, TMAX);
+  float *part = B.get<float>((size_t)rows * GROW), *loss = B.get<float>(steps);
+  if (!st || !w || !m || !v || !XT || !xb || !part || !loss) return plain_fail("allocation failed");
   CK(hipMemcpy(st, states, sizeof(double) * 4 * n, hipMemcpyHostToDevice));
   CK(hipMemcpy(w, params, sizeof(float) * NPARAM, hipMemcpyHostToDevice));
-  CK(hipMemset(g, 0, sizeof(float) * NPARAM)); CK(hipMemset(m, 0, sizeof(float) * NPARAM));
+  CK(hipMemset(m, 0, sizeof(float) * NPARAM));
   CK(hipMemset(v, 0, sizeof(float) * NPARAM));
-  hipLaunchKernelGGL(k_mlp_prepare, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, 0, w, st, n, X, T);
+  hipLaunchKernelGGL(k_mlp_prepare, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, 0, w, st, n, XT);
+  unsigned gather = (batch + 255) / 256;
+  hipLaunchKernelGGL(k_mlp_draw, dim3(gather), dim3(256), 0, 0, XT, xb, batch, n, seed, 0ll);
   for (int k = 0; k < steps; ++k) {
-    CK(hipMemset(loss, 0, sizeof(float)));
-    hipLaunchKernelGGL(k_mlp_sample, dim3((batch + 255) / 256), dim3(256), 0, 0, idx, batch, n, seed, (long long)k);
-    hipLaunchKernelGGL(k_mlp_grad, dim3((batch + 63) / 64), dim3(64), 0, 0, w, X, T, idx, batch, g, loss);
-    hipLaunchKernelGGL(k_mlp_adam, dim3((NTRAIN + 255) / 256), dim3(256), 0, 0, w, g, m, v, k + 1, lr);
-    if (loss_hist) CK(hipMemcpy(&loss_hist[k], loss, sizeof(float), hipMemcpyDeviceToHost));
+    float c1 = (float)(1. - pow((double)0.9f, k + 1)), c2 = (float)(1. - pow((double)0.999f, k + 1));
+    hipLaunchKernelGGL(k_mlp_grad, dim3(rows), dim3(256), 0, 0, w, xb, batch, part);
+    hipLaunchKernelGGL(k_mlp_adam, dim3(ADAM_WG + (k + 1 < steps ? gather : 0)), dim3(256), 0, 0, part, rows, w, m, v,
+                       c1, c2, lr, (float*)nullptr, loss + k, XT, xb, batch, n, seed, (long long)k + 1);
   }
   CK(hipGetLastError());
+  if (loss_hist) CK(hipMemcpy(loss_hist, loss, sizeof(float) * steps, hipMemcpyDeviceToHost));
   CK(hipMemcpy(params, w, sizeof(float) * NPARAM, hipMemcpyDeviceToHost));
   return 0;
 #endif
@@ -3559,18 +3630,17 @@ int gammahip_mlp_grad(const float* params, const double* states, int n, float* g
   using namespace gh::mlp;
   DevBuf B;
   double* st = B.get<double>(4 * (size_t)n);
-  float *w = B.get<float>(NPARAM), *g = B.get<float>(NPARAM), *X = B.get<float>(3 * (size_t)n);
-  float *T = B.get<float>(n), *loss = B.get<float>(1);
-  long long* idx = B.get<long long>(n);
-  if (!st || !w || !g || !X || !T || !loss || !idx) return plain_fail("allocation failed");
-  std::vector<long long> hi(n);
-  for (int k = 0; k < n; ++k) hi[k] = k;
+  float *w = B.get<float>(NPARAM), *g = B.get<float>(NPARAM), *loss = B.get<float>(1);
+  float4* XT = B.get<float4>(n);
+  int rows = std::min(n / TS + 1, TMAX);
+  float* part = B.get<float>((size_t)rows * GROW);
+  if (!st || !w || !g || !XT || !part || !loss) return plain_fail("allocation failed");
   CK(hipMemcpy(st, states, sizeof(double) * 4 * n, hipMemcpyHostToDevice));
   CK(hipMemcpy(w, params, sizeof(float) * NPARAM, hipMemcpyHostToDevice));
-  CK(hipMemcpy(idx, hi.data(), sizeof(long long) * n, hipMemcpyHostToDevice));
-  CK(hipMemset(g, 0, sizeof(float) * NPARAM)); CK(hipMemset(loss, 0, sizeof(float)));
-  hipLaunchKernelGGL(k_mlp_prepare, dim3((n + 255) / 256), dim3(256), 0, 0, w, st, (long long)n, X, T);
-  hipLaunchKernelGGL(k_mlp_grad, dim3((n + 63) / 64), dim3(64), 0, 0, w, X, T, idx, n, g, loss);
+  hipLaunchKernelGGL(k_mlp_prepare, dim3((n + 255) / 256), dim3(256), 0, 0, w, st, (long long)n, XT);
+  hipLaunchKernelGGL(k_mlp_grad, dim3(rows), dim3(256), 0, 0, w, XT, n, part);
+  hipLaunchKernelGGL(k_mlp_adam, dim3(ADAM_WG), dim3(256), 0, 0, part, rows, w, (float*)nullptr, (float*)nullptr, 1.f,
+                     1.f, 0.f, g, loss, (const float4*)nullptr, (float4*)nullptr, 0, 0ll, 0ull, 0ll);
   CK(hipGetLastError());
   CK(hipMemcpy(grad, g, sizeof(float) * NTRAIN, hipMemcpyDeviceToHost));
   CK(hipMemcpy(loss_out, loss, sizeof(float), hipMemcpyDeviceToHost));

@@ -102,6 +102,45 @@ def test_gpu_gradient_matches_cpu_reference():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 31, 33, 257, 8192 + 5, 20000])
+def test_gpu_gradient_at_tile_edges(n):
+    """Batches of one state, either side of a 32-state tile, and with more tiles
+    than workgroups.  FP32 sums of 64 terms in three layers: about
+    3 * 64 * 2^-24 = 1e-5 of each block's norm, times ten for cancellation."""
+    w, st = _params(n=20000)
+    st = st[:n]
+    g, loss = SG.gradient(w, st)
+    lref, gref = R.loss_grad(w.astype(np.float64), R.features(w, st), R.targets(w, st))
+    assert abs(loss - lref) <= 1e-4 * lref
+    for a, b in ((SG.OW1, SG.OB1), (SG.OB1, SG.OW2), (SG.OW2, SG.OB2), (SG.OB2, SG.OW3),
+                 (SG.OW3, SG.OB3), (SG.OB3, SG.ONORM)):
+        assert np.linalg.norm(g[a:b] - gref[a:b]) <= 1e-4 * np.linalg.norm(gref[a:b]), (a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch", [64, 100, 9000])
+def test_gpu_training_steps_match_cpu_reference(batch):
+    """Five Adam steps on the counter stream's minibatches.  A parameter moves by
+    at most about lr = 2e-3 a step whatever its gradient's size, so rounding
+    (1e-4 of the gradient, all of it where the gradient is rounding itself, one
+    entry in a hundred at most) leaves 1e-2 of the 5 * 2e-3 * sqrt(4481) moved."""
+    w, st = _params(n=5000)
+    wg, loss = SG.train(st, steps=5, batch=batch, lr=2e-3, seed=9, params=w)
+    X, T = R.features(w, st), R.targets(w, st)
+    wr, m, v = w.astype(np.float64), 0., 0.
+    for k in range(5):
+        z = (np.arange(batch, dtype=np.uint64) + np.uint64(k * batch + 1)) * np.uint64(0x9E3779B97F4A7C15) + np.uint64(9)
+        z = (z ^ (z >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
+        z = (z ^ (z >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
+        at = ((z ^ (z >> np.uint64(31))) % np.uint64(len(st))).astype(np.int64)
+        lref, g = R.loss_grad(wr, X[at], T[at])
+        assert abs(loss[k] - lref) <= 1e-3 * lref
+        m, v = 0.9 * m + 0.1 * g, 0.999 * v + 0.001 * g * g
+        wr[:SG.ONORM] -= 2e-3 * (m / (1 - 0.9 ** (k + 1))) / (np.sqrt(v / (1 - 0.999 ** (k + 1))) + 1e-8)
+    assert np.linalg.norm(wg - wr) <= 1e-2 * 5 * 2e-3 * np.sqrt(SG.ONORM)
+
+
+@pytest.mark.gpu
 def test_gpu_inference_paths():
     w, st = _params(n=5000)
     X = R.features(w, st)
