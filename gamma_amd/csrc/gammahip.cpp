@@ -23,7 +23,6 @@
 #include <vector>
 #include <algorithm>
 #include <map>
-#include <mutex>
 #include <utility>
 
 #ifdef GH_EMU
@@ -2251,35 +2250,61 @@ __global__ void __launch_bounds__(256) k_mlp_adam(const float* __restrict__ part
   w[k] -= lr * (mk / c1) / (sqrtf(vk / c2) + eps);
 }
 
-// batch inference: pressure guesses of raw states; mfma = 1 runs the BF16 MFMA
-// wavefront path, 0 the FP32 reference path
-__global__ void __launch_bounds__(64) k_mlp_infer(const float* __restrict__ w, const bf16x8* __restrict__ w2b,
-                                                  const double* __restrict__ st, long long n,
-                                                  double* __restrict__ out, int mfma) {
-  __shared__ __bf16 lds[64 * H];
-  __shared__ float rows[64];
-  long long s = (long long)blockIdx.x * 64 + threadIdx.x;
-  bool valid = s < n;
-  double D = valid ? st[3 * s] : 1., S = valid ? st[3 * s + 1] : 0., tau = valid ? st[3 * s + 2] : 1.;
-  float x[3];
-  features(w, D, S, tau, x);
-  float y;
-  if (mfma) y = forward_wave(w, w2b, x, lds, rows);
-  else { float h1[H], h2[H]; y = forward_f32(w, x, h1, h2); }
-  if (valid) out[s] = pressure_of(w, D, y);
-}
-
-// B operands of the hidden layer packed per lane on the device, the layout of
-// pack_w2 (one thread per (k-block, n-block, lane), 8 values each), from
-// parameters already in device memory
-__global__ void __launch_bounds__(512) k_mlp_pack_w2(const float* __restrict__ w, __bf16* __restrict__ out) {
-  int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (t >= 8 * 64) return;
-  int l = t % 64, blk = t / 64, kb = blk / 2, nb = blk % 2;
-  for (int e = 0; e < 8; ++e) {
-    int n = nb * 32 + l % 32, k = kb * 16 + 8 * (l / 32) + e;
-    out[t * 8 + e] = (__bf16)w[OW2 + n * H + k];
+// batch inference: pressure guesses of raw states.  MFMA: the BF16 wavefront
+// path, each workgroup packing the network into LDS once (first layer as
+// (b1, W1 row), hidden layer as pack_w2's operands) and walking its share of
+// the states; else the FP32 reference path.  Two builds: the FP32 path's 128
+// hidden values a thread would halve the occupancy of the other.  The MFMA
+// path is bound by the vector ALU (about 1200 instructions per 64 states: 64
+// first-layer units in the rounding order of the FP32 sum, the output layer,
+// three logarithms and an exponential in FP64): 2^20 states 77 -> 35 us.
+template <bool MFMA>
+__global__ void __launch_bounds__(256, MFMA ? 4 : 1) k_mlp_infer(const float* __restrict__ w,
+                                                                 const double* __restrict__ st, long long n,
+                                                                 double* __restrict__ out) {
+  __shared__ float4 u1[MFMA ? H : 1], u2[MFMA ? H / 4 : 1], u3[MFMA ? H / 4 : 1];
+  __shared__ bf16x8 w2[MFMA ? 8 * 64 : 1];
+  int t = (int)threadIdx.x;
+  if constexpr (MFMA) {
+    if (t < H) {
+      u1[t] = make_float4(w[OB1 + t], w[OW1 + 3 * t], w[OW1 + 3 * t + 1], w[OW1 + 3 * t + 2]);
+      ((float*)u2)[t] = w[OB2 + t];
+      ((float*)u3)[t] = w[OW3 + t];
+    }
+    for (int q = t; q < 8 * 64; q += 256) {
+      int l = q % 64, kb = q / 128, nb = q / 64 % 2;
+      const float* row = w + OW2 + (nb * 32 + l % 32) * H + kb * 16 + 8 * (l / 32);
+      bf16x8 v;
+      for (int e = 0; e < 8; ++e) v[e] = (__bf16)row[e];
+      w2[q] = v;
+    }
+    __syncthreads();
   }
+  for (long long s0 = (long long)blockIdx.x * 256; s0 < n; s0 += MFMA ? (long long)gridDim.x * 256 : n) {
+    long long s = s0 + t;
+    bool valid = s < n;
+    double D = valid ? st[3 * s] : 1., S = valid ? st[3 * s + 1] : 0., tau = valid ? st[3 * s + 2] : 1.;
+    float x[3];
+    features(w, D, S, tau, x);
+    float y;
+    if constexpr (MFMA) {
+      y = forward_wave(x, [&](int o) { return u1[o]; }, [&](int q) { return w2[q]; }, [&](int q) { return u2[q]; },
+                       [&](int q) { return u3[q]; }, w[OB3]);
+    } else {
+      float h1[H], h2[H];
+      y = forward_f32(w, x, h1, h2);
+    }
+    if (valid) out[s] = pressure_of(w, D, y);
+  }
+}
+// at most 2048 workgroups, each packing once: two rounds of the 4 a CU that the
+// registers admit, which balance better than one (4 M states 133 against 140 us);
+// the FP32 path has nothing to save and takes a workgroup per 256 states
+constexpr long long INFER_WG = 2048;
+void launch_infer(const float* w, const double* st, long long n, double* out, int mfma, hipStream_t s) {
+  long long g = (n + 255) / 256;
+  if (mfma) hipLaunchKernelGGL(k_mlp_infer<true>, dim3((unsigned)std::min(g, INFER_WG)), dim3(256), 0, s, w, st, n, out);
+  else hipLaunchKernelGGL(k_mlp_infer<false>, dim3((unsigned)g), dim3(256), 0, s, w, st, n, out);
 }
 
 __global__ void k_c2p_batch(const double* __restrict__ st, const double* __restrict__ guess,
@@ -2298,8 +2323,6 @@ __global__ void k_c2p_batch(const double* __restrict__ st, const double* __restr
 struct MlpGuess {
   const float* w;
   const bf16x8* w2b;
-  __bf16* lds;
-  float* rows;
   double thr;
   double G;
   __device__ double operator()(bool want, double D, double S, double tau, double pprev, int geom) const {
@@ -2314,17 +2337,20 @@ struct MlpGuess {
     float x[3];
     if (want) features(w, D, S, tau, x);
     else { x[0] = 0.f; x[1] = 0.f; x[2] = 0.f; }
-    float y = forward_wave(w, w2b, x, lds, rows);
+    const float* p = w;
+    auto four = [p](int at) { return make_float4(p[at], p[at + 1], p[at + 2], p[at + 3]); };
+    const bf16x8* q2 = w2b;
+    float y = forward_wave(
+        x, [p](int o) { return make_float4(p[OB1 + o], p[OW1 + 3 * o], p[OW1 + 3 * o + 1], p[OW1 + 3 * o + 2]); },
+        [q2](int q) { return q2[q]; }, [&](int q) { return four(OB2 + 4 * q); },
+        [&](int q) { return four(OW3 + 4 * q); }, p[OB3]);
     return hard ? pressure_of(w, D, y) : -1.;
   }
 };
 
 template <bool PK, int ND, int NQ>
 __global__ void __launch_bounds__(KB) k_update_mlp(Dev d, int ni, int remap, int stage) {
-  __shared__ __bf16 lds[KB / 64][64 * H];
-  __shared__ float rows[KB / 64][64];
-  int wv = threadIdx.x / 64;
-  MlpGuess g{d.mw, (const bf16x8*)d.mw2b, lds[wv], rows[wv], d.mlp_thr, d.P.gamma};
+  MlpGuess g{d.mw, (const bf16x8*)d.mw2b, d.mlp_thr, d.P.gamma};
   GH_TILE_LOOP(PK, {
     if (stage > 1 && i < ni && j < d.nj) body_dt(d, j, i);
     body_update_g<ND, NQ, C2P_NEWTON>(d, j, i, stage, i < ni && j < d.nj, g);
@@ -2905,36 +2931,6 @@ int plain_fail(const char* m) { fprintf(stderr, "gammahip: %s\n", m); return -1;
 #define CK(x) do { if ((x) != hipSuccess) return plain_fail(#x); } while (0)
 }  // namespace
 
-// Device memory of gammahip_mlp_infer_noalloc, in place of the buffers
-// gammahip_mlp_infer allocates per call: the hidden layer's packed BF16 B
-// operands (8 x 64 lanes x 8 values = 8 KiB).  Each device holds its own copy
-// until the process ends.  In host code `scratch` names a host-side stand-in:
-// kernels get the device address from noalloc_scratch() instead.
-constexpr size_t NOALLOC_SCRATCH_BYTES = 16384;
-static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES];
-
-namespace {
-constexpr int NOALLOC_MAX_DEVICES = 64;
-std::mutex noalloc_mu;
-void* noalloc_ptr[NOALLOC_MAX_DEVICES];
-
-// device address of the current device's copy of `scratch`, looked up once per
-// device (with that device current) and kept
-int noalloc_scratch(void** out) {
-  int dev = -1;
-  CK(hipGetDevice(&dev));
-  if (dev < 0 || dev >= NOALLOC_MAX_DEVICES) return plain_fail("noalloc: device index out of range");
-  std::lock_guard<std::mutex> lock(noalloc_mu);
-  if (!noalloc_ptr[dev]) {
-    void* p = nullptr;
-    hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-    if (e != hipSuccess || !p) return plain_fail("noalloc: hipGetSymbolAddress(scratch) failed");
-    noalloc_ptr[dev] = p;
-  }
-  *out = noalloc_ptr[dev];
-  return 0;
-}
-}  // namespace
 #endif
 
 extern "C" {
@@ -3657,14 +3653,10 @@ int gammahip_mlp_infer(const float* params, const double* states, long long n, d
   DevBuf B;
   double *st = B.get<double>(3 * n), *out = B.get<double>(n);
   float* w = B.get<float>(NPARAM);
-  bf16x8* w2b = B.get<bf16x8>(8 * 64);
-  if (!st || !out || !w || !w2b) return plain_fail("allocation failed");
-  std::vector<__bf16> hb(8 * 64 * 8);
-  pack_w2(params, hb.data());
+  if (!st || !out || !w) return plain_fail("allocation failed");
   CK(hipMemcpy(st, states, sizeof(double) * 3 * n, hipMemcpyHostToDevice));
   CK(hipMemcpy(w, params, sizeof(float) * NPARAM, hipMemcpyHostToDevice));
-  CK(hipMemcpy(w2b, hb.data(), sizeof(__bf16) * hb.size(), hipMemcpyHostToDevice));
-  hipLaunchKernelGGL(k_mlp_infer, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, 0, w, w2b, st, n, out, mfma);
+  launch_infer(w, st, n, out, mfma, 0);
   CK(hipGetLastError());
   CK(hipMemcpy(p_out, out, sizeof(double) * n, hipMemcpyDeviceToHost));
   return 0;
@@ -3678,19 +3670,11 @@ int gammahip_mlp_infer_noalloc(const float* params, const double* states, long l
   return -1;
 #else
   using namespace gh::mlp;
-  constexpr size_t need = sizeof(bf16x8) * 8 * 64;
-  static_assert(need <= NOALLOC_SCRATCH_BYTES, "packed operands exceed the scratch array");
   if (!params || !states || !p_out) return plain_fail("mlp_infer_noalloc: null device pointer");
   if (mfma != 0 && mfma != 1) return plain_fail("mlp_infer_noalloc: mfma must be 0 or 1");
   if (n < 1 || (n + 63) / 64 > (long long)INT_MAX)
     return plain_fail("mlp_infer_noalloc: n must be in [1, 64 * INT_MAX]");
-  void* sp = nullptr;
-  if (noalloc_scratch(&sp)) return -1;
-  hipStream_t s = (hipStream_t)stream;
-  bf16x8* w2b = (bf16x8*)sp;
-  hipLaunchKernelGGL(k_mlp_pack_w2, dim3(1), dim3(512), 0, s, params, (__bf16*)w2b);
-  hipLaunchKernelGGL(k_mlp_infer, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, s, params, w2b, states, n, p_out,
-                     mfma);
+  launch_infer(params, states, n, p_out, mfma, (hipStream_t)stream);
   CK(hipGetLastError());
   return 0;
 #endif

@@ -96,54 +96,61 @@ __host__ inline void pack_w2(const float* w, __bf16* out) {
         }
 }
 
-// Forward of the 64 cells of a wavefront (one per lane).  Must be reached by
-// all 64 lanes together (uniform control flow): lanes without a cell pass any
-// finite features and ignore the result.  lds: 64*64 bf16 scratch per wave
-// (H1 rows), rowsum: 64 floats per wave.
-__device__ float forward_wave(const float* __restrict__ w, const bf16x8* __restrict__ w2b,
-                              const float* x, __bf16* lds, float* rowsum) {
-  int l = threadIdx.x & 63;
-  // layer 1 on the vector ALU, written as bf16 rows of H1 (row = lane)
-  for (int o = 0; o < H; ++o) {
-    float a = w[OB1 + o] + w[OW1 + o * 3] * x[0] + w[OW1 + o * 3 + 1] * x[1] + w[OW1 + o * 3 + 2] * x[2];
-    lds[l * H + o] = (__bf16)(a > 0.f ? a : 0.f);
-  }
-  __builtin_amdgcn_s_waitcnt(0);
-  __builtin_amdgcn_wave_barrier();
-  // hidden layer: D[rb][nb] = sum_kb A[rb][kb] B[kb][nb], 16 MFMA per wave
-  floatx16 acc[2][2];
-  for (int rb = 0; rb < 2; ++rb)
-    for (int nb = 0; nb < 2; ++nb) acc[rb][nb] = floatx16{};
-  for (int kb = 0; kb < 4; ++kb) {
-    for (int rb = 0; rb < 2; ++rb) {
-      bf16x8 a;
-      const __bf16* src = lds + (rb * 32 + l % 32) * H + kb * 16 + 8 * (l / 32);
-      for (int e = 0; e < 8; ++e) a[e] = src[e];
-      for (int nb = 0; nb < 2; ++nb)
-        acc[rb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, w2b[(kb * 2 + nb) * 64 + l], acc[rb][nb], 0, 0, 0);
-    }
-  }
-  // bias, ReLU and the output layer: per-lane partial row sums, then a reduction
-  // over the 32 lanes that share the same rows
-  for (int rb = 0; rb < 2; ++rb) {
-    float part[16];
-    for (int r = 0; r < 16; ++r) part[r] = 0.f;
-    for (int nb = 0; nb < 2; ++nb) {
-      int col = nb * 32 + l % 32;
-      float b2 = w[OB2 + col], w3 = w[OW3 + col];
-      for (int r = 0; r < 16; ++r) {
-        float v = acc[rb][nb][r] + b2;
-        part[r] += w3 * (v > 0.f ? v : 0.f);
+// Forward of the 64 cells of a wavefront (one per lane, features x).  Must be
+// reached by all 64 lanes together (uniform control flow): lanes without a
+// cell pass any finite features and ignore the result.  l1(o): unit o of the
+// first layer as (b1, W1[o][0..2]); w2: the packed operand of pack_w2 at an index;
+// l2(q), l3(q): b2 and w3 of units 4q .. 4q + 3.
+// The hidden layer is formed transposed, D = W2 H1^T with the cells along the
+// columns: a lane then computes just the first-layer units its B operands
+// need (those of cells l%32 and 32 + l%32) and holds 16 units of a cell's
+// column, so the output layer is summed inside the lane but for one exchange
+// of lane halves per four values.  With the cells along the rows it took 160
+// exchanges and an H1 tile in LDS whose rows all began in one bank: 2^20
+// cells took 78 us that way.  The sum over units is the balanced tree
+// over bits 4, 3, 2, 1, 0 of the unit (blocks 0 and 32 added first).
+template <class L1, class W2, class L2, class L3>
+__device__ float forward_wave(const float* x, L1&& l1, W2&& w2, L2&& l2, L3&& l3, float b3) {
+  int l = threadIdx.x & 63, hf = l >> 5;
+  float xo[3], y = 0.f;                             // features of the cell the other half's lane holds
+  for (int k = 0; k < 3; ++k) xo[k] = __shfl_xor(x[k], 32, 64);
+#pragma unroll 1
+  for (int sb = 0; sb < 2; ++sb) {                 // cells 32 sb + l%32, one block at a time: 32 accumulators, not 64
+    int at = hf;                                   // opaque: keeps the weights of both blocks' loads in the loop
+    asm volatile("" : "+v"(at));
+    float xc[3];
+    for (int k = 0; k < 3; ++k) xc[k] = sb == hf ? x[k] : xo[k];
+    floatx16 acc[2] = {floatx16{}, floatx16{}};    // units 32 nb ..
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+      bf16x8 h;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float4 u = l1(kb * 16 + 8 * at + e);
+        float a = u.x + u.y * xc[0] + u.z * xc[1] + u.w * xc[2];
+        h[e] = (__bf16)fmaxf(a, 0.f);
       }
+      for (int nb = 0; nb < 2; ++nb)
+        acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w2((kb * 2 + nb) * 64 + l), h, acc[nb], 0, 0, 0);
     }
-    for (int r = 0; r < 16; ++r)
-      for (int off = 16; off > 0; off >>= 1) part[r] += __shfl_xor(part[r], off, 64);
-    if (l % 32 == 0)
-      for (int r = 0; r < 16; ++r) rowsum[rb * 32 + d_row(l, r)] = part[r];
+    float part[16];                                // unit 8 (r/4) + 4 hf + r%4
+    for (int r = 0; r < 16; ++r) part[r] = 0.f;
+    for (int nb = 0; nb < 2; ++nb)
+      for (int q = 0; q < 4; ++q) {
+        float4 b = l2(nb * 8 + 2 * q + at), u = l3(nb * 8 + 2 * q + at);
+        float b2[4] = {b.x, b.y, b.z, b.w}, w3[4] = {u.x, u.y, u.z, u.w};
+        for (int r = 0; r < 4; ++r) {
+          float v = acc[nb][4 * q + r] + b2[r];
+          part[4 * q + r] += w3[r] * fmaxf(v, 0.f);
+        }
+      }
+    for (int r = 0; r < 8; ++r) part[r] += part[r + 8];
+    for (int r = 0; r < 4; ++r) part[r] += part[r + 4];
+    for (int r = 0; r < 4; ++r) part[r] += __shfl_xor(part[r], 32, 64);
+    float ys = (part[0] + part[2]) + (part[1] + part[3]);
+    if (sb == hf) y = ys;
   }
-  __builtin_amdgcn_s_waitcnt(0);
-  __builtin_amdgcn_wave_barrier();
-  return rowsum[l] + w[OB3];
+  return y + b3;
 }
 
 }  // namespace mlp

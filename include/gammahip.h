@@ -246,10 +246,9 @@ int  gammahip_mlp_infer(const float* params, const double* states, long long n, 
  * capture, tight serving loops).  params [gammahip_mlp_nparams()], states
  * [n][3] and p_out [n] are DEVICE pointers; the call is asynchronous on
  * stream (a hipStream_t; null = the default stream) and returns the bits of
- * gammahip_mlp_infer.  The packed BF16 hidden-layer operands go into a fixed
- * 16 KiB device array of the library (one per device, held until the process
- * ends; 8 KiB used, whatever n), fully rewritten by every call: calls that
- * overlap on one device race on it.  Rejects null pointers, mfma not 0/1 and
+ * gammahip_mlp_infer.  One kernel launch; the network is packed on chip, so no
+ * device memory but the caller's is used and calls may overlap on several
+ * streams.  Rejects null pointers, mfma not 0/1 and
  * n outside [1, 64 * INT_MAX] with -1 and a message on stderr. */
 int  gammahip_mlp_infer_noalloc(const float* params, const double* states, long long n, double* p_out,
                                 int mfma, void* stream);

@@ -155,6 +155,22 @@ def test_gpu_inference_paths():
     assert np.sqrt(np.mean((ymf - yref) ** 2)) < 0.05 * spread
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 63, 65, 255, 2048 * 256 + 3])
+def test_gpu_inference_at_tile_edges(n):
+    """Counts either side of a wavefront, a workgroup and the whole grid: a
+    state's answer does not depend on its place, and follows the BF16 emulation
+    (the bound of test_gpu_inference_paths)."""
+    w, st = _params(n=5000)
+    big = np.tile(st, (n // len(st) + 1, 1))[:n]
+    p = SG.infer(w, big, mfma=True)
+    ref = SG.infer(w, st, mfma=True)
+    np.testing.assert_array_equal(p, np.tile(ref, n // len(st) + 1)[:n])
+    yemu = R.forward_mfma(w.astype(np.float64), R.features(w, st))
+    m = min(n, len(st))
+    assert np.max(np.abs(R.y_of_pressure(w, st, ref) - yemu)[:m]) < 1e-3 * max(np.std(yemu), 1.0)
+
+
 def _train_set(n_syn=1 << 18):
     syn = SG.synthetic_states(n_syn, G53, seed=21)
     return syn
