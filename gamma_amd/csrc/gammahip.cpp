@@ -1049,29 +1049,38 @@ GH_HD void body_init_gammas(const Dev& d, int j, int i) {
 // 2d.cpp:609-832) with the checkCellForRegrid hooks of the setups.
 enum { RG_SKIP = 0, RG_MERGE = 1, RG_SPLIT = 2 };
 
+// the aspect-ratio rule (2DST.cpp:304-322) of a cell of width dx
+GH_HD int rg_rule_ar(const Dev& d, double dx, double dy) {
+  double ar = dx / dy;
+  if (ar > d.rg[0]) return RG_SPLIT;
+  if (ar < d.rg[1]) return RG_MERGE;
+  return RG_SKIP;
+}
+// the Blandford-McKee rule (BM1D.cpp:277-319) of a cell of width dx and Lorentz
+// factor lf, dist cells past the shock, on a track of outer radius rOut.  Few
+// cells lie near the two bounds: where ar lf^(3/2) in plain arithmetic (within
+// 1e-15) lies between them by more than 1e-9 the correctly rounded power
+// decides nothing else and is not formed.
+GH_HD int rg_rule_bm(const Dev& d, double dx, double lf, double dist, double rOut) {
+  double dth = d.rg[2], target = d.rg[4];
+  double ar = dx / (rOut * dth);
+  if (0 < dist && dist < 10) ar *= 10;
+  double hi = d.rg[0] * target, lo = d.rg[1] * target, q = ar * (lf * sqrt(lf));
+  if (hi > 0. && (lo == 0. || lo > 1.e-290) && q > lo * (1. + 1.e-9) && q < hi * (1. - 1.e-9)) return RG_SKIP;
+  if (ar > d.rg[0] * target / gh_pow(lf, 3. / 2.)) return RG_SPLIT;
+  if (ar < d.rg[1] * target / gh_pow(lf, 3. / 2.)) return RG_MERGE;
+  return RG_SKIP;
+}
 template <int ND, int NQ>
 GH_HD int rg_check(const Dev& d, int j, int i, double iS) {
   long long k = CI(d, j, i);
   int mode = d.trg[j];
-  if (mode == RG_AR2D) {
-    double ar = d.cdx[k] / d.tdy[j];
-    if (ar > d.rg[0]) return RG_SPLIT;
-    if (ar < d.rg[1]) return RG_MERGE;
-    return RG_SKIP;
-  }
+  if (mode == RG_AR2D) return rg_rule_ar(d, d.cdx[k], d.tdy[j]);
   if (mode == RG_BM1D) {
     int nt = d.ntrack[j], iR = nt - d.ngst;
-    double dth = d.rg[2], target = d.rg[4];
-    double rOut = d.cx[CI(d, j, iR - 1)];
-    double ar = d.cdx[k] / (rOut * dth);
-    double dist = i - iS;
-    if (0 < dist && dist < 10) ar *= 10;
     double p[NQ];
     load_v<ND, NQ>(d, d.prim, k, p);
-    double lf = lfac<ND, NQ>(p);
-    if (ar > d.rg[0] * target / gh_pow(lf, 3. / 2.)) return RG_SPLIT;
-    if (ar < d.rg[1] * target / gh_pow(lf, 3. / 2.)) return RG_MERGE;
-    return RG_SKIP;
+    return rg_rule_bm(d, d.cdx[k], lfac<ND, NQ>(p), i - iS, d.cx[CI(d, j, iR - 1)]);
   }
   if (mode == RG_USER) {
     double p[NQ];
@@ -1269,19 +1278,13 @@ GH_HD void body_rg_init(const Dev& d, int j, int i) {
   d.tlast[j] = -1;
   d.tiS[j] = d.ngst;        // iLbnd + 1
 }
-// In the plain launch (a thread for every slot of the track) the threads take
-// the cells from the far end of the track (cell nax-1-i), so that the
-// wavefronts dispatched first hold the largest indices; a thread whose
-// candidate does not exceed the maximum already stored (it only grows; a
-// stale read is lower) leaves out its atomic: the same maximum with far fewer
-// same-address atomics per track.  The packed launch walks the live cells
-// only, in their own order.
+// (init, shock position, screen and body_rg_apply are the sequential form that
+// the CPU build runs; the GPU's is wg_screen and k_regrid)
 GH_HD void body_rg_shockpos(const Dev& d, int j, int i) {
   if (!active_track(d, j) || d.trg[j] != RG_BM1D) return;
-  if (!d.packed) i = d.nax - 1 - i;
   int nt = d.ntrack[j], iL = d.ngst - 1, iR = nt - d.ngst;
   if (i < iL + 1 || i > iR - 1) return;
-  if (d.prim[PPP * d.cs + CI(d, j, i)] > 1.5 * d.rg[3] && i > d.tiS[j]) GH_ATOMIC_MAX(&d.tiS[j], i);
+  if (d.prim[PPP * d.cs + CI(d, j, i)] > 1.5 * d.rg[3] && i > d.tiS[j]) d.tiS[j] = i;
 }
 template <int ND, int NQ>
 GH_HD void body_rg_screen(const Dev& d, int j, int i) {
@@ -1306,9 +1309,9 @@ GH_HD void body_rg_screen(const Dev& d, int j, int i) {
 // none past tlast.  (CIRC_REGRID_ and the user rule read more of the track:
 // never stopped early.)
 struct RgStop { int tl, nt0; double iS0, rOut0; bool on; };
-GH_HD RgStop rg_stop_init(const Dev& d, int j, double iS) {
+GH_HD RgStop rg_stop_init(const Dev& d, int j, double iS, int tl) {
   RgStop s;
-  s.tl = d.tlast[j];
+  s.tl = tl;
   s.nt0 = d.ntrack[j];
   s.iS0 = iS;
   s.rOut0 = d.cx[CI(d, j, s.nt0 - d.ngst - 1)];
@@ -1358,7 +1361,7 @@ GH_HD void body_rg_apply(const Dev& d, int j, int i0) {
   double iS = bm ? (double)d.tiS[j] : 0.;
   int is = -1, ib = -1;
   if (d.circ) rg_victims<ND, NQ>(d, j, &is, &ib);
-  RgStop stop = rg_stop_init(d, j, iS);
+  RgStop stop = rg_stop_init(d, j, iS, d.tlast[j]);
   int last_mod = -1;                       // the last cell a split or merge wrote
   for (; i <= d.ntrack[j] - d.ngst - 1; ++i) {
     if (rg_stop(d, j, stop, i, last_mod, iS)) break;
@@ -1571,8 +1574,6 @@ __global__ void __launch_bounds__(KB) k_nb(Dev d, int ni, int remap) {
 GH_KERNEL2P((), k_f1_shock, body_f1_shock)
 GH_KERNEL2(k_shock_reset, body_shock_reset)
 GH_KERNEL2(k_shock_detect, body_shock_detect)
-GH_KERNEL2(k_rg_init, body_rg_init)
-GH_KERNEL2P((), k_rg_shockpos, body_rg_shockpos)
 GH_KERNEL2(k_advance_time, body_advance_time)
 template <int ND, int NQ> GH_KERNEL2(k_ghost_mv, (body_ghost_mv<ND, NQ>))
 // updateGhosts of a 2D grid in one launch: workgroups [0, ncopy) copy the
@@ -1680,7 +1681,6 @@ __global__ void __launch_bounds__(KB, (update_waves<ND, NQ, W, GEO>())) k_update
 }
 GH_KERNEL2P((, int ND, int NQ), k_inject, (body_inject<ND, NQ>))
 template <int ND, int NQ> GH_KERNEL2(k_init_gammas, (body_init_gammas<ND, NQ>))
-GH_KERNEL2P((, int ND, int NQ), k_rg_screen, (body_rg_screen<ND, NQ>))
 
 // Tile list of the packed launch: ceil(ntrack / bs) chunks of every track, in
 // track order (one workgroup; block-wide scan of the per-thread counts).
@@ -1964,21 +1964,83 @@ __device__ void wg_merge(const Dev& d, int j, long long b, int i, int* s_left) {
   }
   __syncthreads();
 }
+// One pass over the workgroup's track ahead of the loop: every active cell's
+// decision (rgflag), the shock index and the first and last flagged cell, all
+// of body_rg_shockpos and body_rg_screen.  A decision depends on the shock
+// index only in the nine cells past it, so the cells are read once, judged
+// without that window, and the window judged again when the index is known.
+// One launch instead of four (clear, shock position, screen, loop): a regrid
+// without actions takes 8 instead of 17 us on one 4000-cell track, 39 instead
+// of 62 us on 256 tracks of 512-16384 cells, 30 us either way on 2048 x 2048.
 template <int ND, int NQ>
-__global__ void __launch_bounds__(RGB) k_rg_apply(Dev d) {
+__device__ bool wg_screen(const Dev& d, int j, bool bm, int* red, int* i0, int* i1, double* iS) {
+  int nt = d.ntrack[j], iL = d.ngst - 1, iR = nt - d.ngst, t = (int)threadIdx.x;
+  long long b = CI(d, j, 0);
+  double thr = 1.5 * d.rg[3];
+  auto flag = [&](int i, int a) {
+    bool ok = (a == RG_SPLIT && nt < d.nax - 1) || (a == RG_MERGE && nt > 2 * d.ngst + 2);
+    d.rgflag[b + i] = ok ? 1 : 0;
+    return ok ? 1 : 0;
+  };
+  int any = 0, best = iL + 1, mode = d.trg[j];
+  if (mode == RG_USER) {
+    for (int i = iL + 1 + t; i <= iR - 1; i += RGB) any |= flag(i, rg_check<ND, NQ>(d, j, i, HUGE_VAL));
+  } else {
+    // U cells of a thread at a time, all read before the first is judged
+    constexpr int U = 4;
+    double rOut = d.cx[b + iR - 1], dy = d.tdy[j];
+    for (int i = iL + 1 + t; i <= iR - 1; i += U * RGB) {
+      double dx[U], pp[U], p[U][NQ];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        long long k = b + (i + u * RGB <= iR - 1 ? i + u * RGB : i);
+        dx[u] = d.cdx[k];
+        if (bm) {
+          pp[u] = d.prim[PPP * d.cs + k];
+          p[u][UU1] = d.prim[UU1 * d.cs + k];
+          if (ND == 2) p[u][UU2] = d.prim[UU2 * d.cs + k];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        int m = i + u * RGB;
+        if (m > iR - 1) break;
+        if (bm && pp[u] > thr) best = m;
+        any |= flag(m, bm ? rg_rule_bm(d, dx[u], lfac<ND, NQ>(p[u]), -HUGE_VAL, rOut) : rg_rule_ar(d, dx[u], dy));
+      }
+    }
+  }
+  *iS = 0.;
+  if (bm) {
+    int s = wg_reduce<true>(best, red);
+    *iS = (double)s;
+    int m = s + 1 + t;
+    if (t < 9 && m <= iR - 1) any |= flag(m, rg_check<ND, NQ>(d, j, m, *iS));
+  }
+  if (!wg_reduce<true>(any, red)) return false;
+  int f = INT_MAX, l = -1;
+  for (int i = iL + 1 + t; i <= iR - 1; i += RGB)
+    if (d.rgflag[b + i]) { f = f < i ? f : i; l = i; }
+  *i0 = wg_reduce<false>(f, red);
+  *i1 = wg_reduce<true>(l, red);
+  __syncthreads();
+  return *i1 >= 0;
+}
+template <int ND, int NQ>
+__global__ void __launch_bounds__(RGB) k_regrid(Dev d) {
   __shared__ int red[RGB];
   __shared__ double rv[RGB];
   __shared__ int s_act;
   int j = blockIdx.x;
-  if (!active_track(d, j)) return;
-  int i = d.tfirst[j];
-  if (i == INT_MAX) return;
+  if (!active_track(d, j) || d.trg[j] == RG_NONE) return;
   bool bm = d.trg[j] == RG_BM1D;
   long long b = CI(d, j, 0);
-  double iS = bm ? (double)d.tiS[j] : 0.;    // as body_rg_apply
+  int i, tl;
+  double iS;
+  if (!wg_screen<ND, NQ>(d, j, bm, red, &i, &tl, &iS)) return;
   int is = -1, ib = -1;
   if (d.circ) wg_victims<ND, NQ>(d, j, rv, red, &is, &ib);
-  RgStop stop = rg_stop_init(d, j, iS);
+  RgStop stop = rg_stop_init(d, j, iS, tl);
   int last_mod = -1;                       // the last cell a split or merge wrote
   for (;;) {
     int nt = d.ntrack[j];
@@ -2843,13 +2905,13 @@ struct Pipe {
   static void regrid(gammahip_ctx* c) {
     Dev& d = c->d;
     if (!d.rg_mode) return;
-    L2(c, KSEL(body_rg_init, k_rg_init), d.nj, 1);
-    if (d.rg_mode & (1 << RG_BM1D)) L2P(c, body_rg_shockpos, k_rg_shockpos, (), d.nj, d.nax);
-    L2P(c, (body_rg_screen<ND, NQ>), k_rg_screen, (, ND, NQ), d.nj, d.nax);
 #ifdef GH_EMU
+    L2(c, body_rg_init, d.nj, 1);
+    if (d.rg_mode & (1 << RG_BM1D)) L2(c, body_rg_shockpos, d.nj, d.nax);
+    L2(c, (body_rg_screen<ND, NQ>), d.nj, d.nax);
     for (int j = 0; j < d.nj; ++j) body_rg_apply<ND, NQ>(d, j, 0);
 #else
-    hipLaunchKernelGGL((k_rg_apply<ND, NQ>), dim3(d.nj), dim3(RGB), 0, c->stream, d);
+    hipLaunchKernelGGL((k_regrid<ND, NQ>), dim3(d.nj), dim3(RGB), 0, c->stream, d);
 #endif
   }
   static void apply(gammahip_ctx* c, int what) {
