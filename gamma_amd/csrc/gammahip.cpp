@@ -55,6 +55,13 @@ enum { BND_NONE = 0, BND_BM = 1, BND_USER = 2 };
 enum { RG_NONE = 0, RG_AR2D = 1, RG_BM1D = 2, RG_USER = 3 };
 
 constexpr int DT_CH = 1024;   // cells per workgroup of the per-track dt minimum
+// A tile is S1B - 1 cells: thread t takes face and cell tile*(S1B-1) + t - 1,
+// thread 0 only the left face of the tile's first cell, which the tile before
+// it owns.  The faces meet their right-hand cells through LDS.  One wavefront
+// a workgroup: nothing to wait for at the barrier and a track spread over the
+// most CUs (24 tracks of 512-2048 cells 135 us a step, against 165 and 138 with
+// 128 and 256 threads; 256 tracks 770 against 804 and 809).
+constexpr int S1B = 64, S1C = S1B - 1;
 
 // ---------------------------------------------------------------------------
 // device view (passed by value to every kernel)
@@ -76,7 +83,9 @@ struct Dev {
   double *tvin, *tvout, *tbm, *ty, *tdy, *tdt, *tt, *tmin;
   double *tpart;           // [nj][dtch] dt minimum of each chunk of DT_CH cells of each track
   int dtch;                // chunks per track: ceil(nax / DT_CH)
+  int s1ch;                // 1D: tiles per track of the stage passes, ceil(nax / S1C); tpart is [nj][s1ch] there
   // cells
+  double *primn, *cxn, *cdxn;   // 1D: the stage passes' output state (swapped with prim, cx, cdx)
   double *prim, *cx, *cdx, *dtloc, *U0, *dV0, *gmv, *gf1, *gf1n, *sd, *pspec;
   int *shk, *nbdj, *nbdlo, *nbdcnt, *nbuj, *nbulo, *nbucnt, *f1off, *f1tot;
   int *f1own;              // [nj][fcap] cell owning each F1 face slot
@@ -305,15 +314,15 @@ GH_HD void body_ghost_mv(const Dev& d, int j, int kk) { body_ghost_mv_src<ND, NQ
 // ---------------------------------------------------------------------------
 // Grid::movDir_ComputeLambda + updateKinematics + computeFluxes, MV faces
 // (1d.cpp:370-461, 731-776; 2d.cpp:451-490, 835-888; hllc.cpp:12-39)
-template <int ND, int NQ, bool SHK>
-GH_HD void body_faces_s(const Dev& d, int j, int i) {
-  int nt = d.ntrack[j];
-  if (i > nt - 2) return;
+// Face i (0 <= i <= nt - 2) of track j: reconstructed states, signal speeds,
+// face speed and flux times area; in 2D stores the cells' MV gradients
+template <int ND, int NQ>
+GH_HD void face_flux(const Dev& d, int j, int i, int nt, double* pL, double* pR, Waves& w, double& v, double* fl) {
   int geom = d.tgeom[j];
   double G = d.P.gamma;
   long long k = CI(d, j, i);
   double xf = d.fx[k];
-  double pL[NQ], cL[NQ], pR[NQ], cR[NQ];
+  double cL[NQ], cR[NQ];
   // side fluxes: at the track ends the cells' own states (sweep radius), inside
   // the reconstructed states at the face
   bool edge = d.pc || i == 0 || i == nt - 2;     // piecewise constant: 1d.cpp:378-381
@@ -348,8 +357,8 @@ GH_HD void body_faces_s(const Dev& d, int j, int i) {
     prim2cons<ND, NQ>(pL, cL, xf, geom, G, d.P.synge);
     prim2cons<ND, NQ>(pR, cR, xf, geom, G, d.P.synge);
   }
-  Waves w = lambdas<ND, NQ>(pL, cL, pR, cR, 0, xf, geom, G);
-  double v = d.P.vi * w.lS;
+  w = lambdas<ND, NQ>(pL, cL, pR, cR, 0, xf, geom, G);
+  v = d.P.vi * w.lS;
   if (d.tkin[j] == KIN_FIXED) {
     for (int n = 0; n < d.ngst; ++n) {
       if (i == n) v = d.tvin[j];
@@ -361,11 +370,19 @@ GH_HD void body_faces_s(const Dev& d, int j, int i) {
   }
   Trig T = trig_at<ND>(d, j);
   double dA = face_area<ND>(0, xf, d.tdy[j], geom, T.s_y, T.s_hdy);
-  double fl[NQ];
   hllc_flux_lazy<ND, NQ>(pL, cL, pR, cR, w, v, dA, 0, xf, geom, [&](bool right, double* f) {
     if (right) state2flux<ND, NQ>(pR, cR, f, 0, rR, geom);
     else state2flux<ND, NQ>(pL, cL, f, 0, rL, geom);
   }, fl);
+}
+template <int ND, int NQ, bool SHK>
+GH_HD void body_faces_s(const Dev& d, int j, int i) {
+  int nt = d.ntrack[j];
+  if (i > nt - 2) return;
+  long long k = CI(d, j, i);
+  double pL[NQ], pR[NQ], fl[NQ], v;
+  Waves w;
+  face_flux<ND, NQ>(d, j, i, nt, pL, pR, w, v, fl);
   if (fl[0] != fl[0]) GH_ATOMIC_ADD(cnt_at(d, CNT_NANFLUX), 1ull);
   d.fv[k] = v;
   d.flL[k] = w.lL;
@@ -373,7 +390,7 @@ GH_HD void body_faces_s(const Dev& d, int j, int i) {
   store_v<ND, NQ>(d, d.fflux, k, fl);
   if (SHK) {
     double ps = -1.e300;
-    double Sd = shock_sd<ND, NQ>(pL, pR, 0, false, G, &ps, d.vpspec);
+    double Sd = shock_sd<ND, NQ>(pL, pR, 0, false, d.P.gamma, &ps, d.vpspec);
     d.sd[k] = fmax(d.sd[k], Sd);
     if (ps > d.pspec[k]) d.pspec[k] = ps;
   }
@@ -387,14 +404,16 @@ GH_HD void body_faces(const Dev& d, int j, int i) {
 
 // Cell::update_dt, MV candidates (cell.cpp:47-99)
 // the smaller of the dt candidates cell k's two MV faces give it
-GH_HD double dt_cand(const Dev& d, long long k) {
-  double a = d.cdx[k];
-  double l, v, dtL, dtR;
-  l = d.flR[k - 1]; v = d.fv[k];
-  if (l > v) dtL = a / (l - v); else dtL = 1.e15;
-  l = d.flL[k]; v = d.fv[k - 1];
-  if (l < v) dtR = a / (v - l); else dtR = 1.e15;
+// (cell width a; left face's speed vl and right-going signal lR; right face's
+// speed vr and left-going signal lL)
+GH_HD double dt_cand(double a, double vl, double lR, double vr, double lL) {
+  double dtL, dtR;
+  if (lR > vr) dtL = a / (lR - vr); else dtL = 1.e15;
+  if (lL < vl) dtR = a / (vl - lL); else dtR = 1.e15;
   return fmin(dtL, dtR);
+}
+GH_HD double dt_cand(const Dev& d, long long k) {
+  return dt_cand(d.cdx[k], d.fv[k - 1], d.flR[k - 1], d.fv[k], d.flL[k]);
 }
 GH_HD void body_dt(const Dev& d, int j, int i) {
   int nt = d.ntrack[j];
@@ -870,51 +889,24 @@ inline void capture_c2p(double D, double S, double tau, double pprev, double p, 
 }
 #endif
 
-// GEO: the grid's geometry when fixed at compile time (2D grids have one;
-// -1: the track's, as 1D ensembles mix them)
-template <int ND, int NQ, int SV, class GuessT, int GEO = -1>
-GH_HD void body_update_g(const Dev& d, int j, int i, int stage, bool valid, const GuessT& guess) {
-  bool run = valid && active_track(d, j);
-  int nt = run ? d.ntrack[j] : 0;
-  run = run && i < nt;
-  int iL = d.ngst - 1, iR = nt - d.ngst;
-  int geom = GEO >= 0 ? GEO : run ? d.tgeom[j] : 0;
+// Cell::update of cell (j, i) (cell.cpp:102-127), then in stages 2 and 3 the
+// RK3 average with the state at the start of the step: cons2prim after each.
+// xnL, xnR: its faces advanced by dt; xaL, xaR: the same averaged (stages 2,
+// 3); mv(fa, fb) gives the fluxes through them.  p and (*cxo, *cdxo): the new
+// state.  Called by every thread (cell = false for threads without one), as
+// the starting-pressure provider may use wavefront-wide operations.
+template <int ND, int NQ, int SV, class GuessT, class MvFlux>
+GH_HD void cell_advance(const Dev& d, int j, int i, long long k, int geom, int stage, double dt, bool cell,
+                        double xnL, double xnR, double xaL, double xaR, const MvFlux& mv, const GuessT& guess,
+                        double* p, double* cxo, double* cdxo) {
   double G = d.P.gamma;
-  double dt = run ? d.tdt[j] : 0.;
   double w0 = stage == 2 ? 3. / 4. : 1. / 3.;
   double w1 = stage == 2 ? 1. / 4. : 2. / 3.;
-  long long k = run ? CI(d, j, i) : 0;
-  bool cell = false;
-  double p[NQ], U[NQ];
+  double U[NQ];
   for (int q = 0; q < NQ; ++q) { p[q] = 0.; U[q] = 0.; }
-  double xnL = 0., xnR = 0., cxn = 0., cdxn = 0., r1 = 0.;
+  double cxn = 0., cdxn = 0., r1 = 0.;
   Geo g2 = {};
-  if (run) {
-    if (i <= nt - 2) {
-      double xo = d.fx[k];
-      double xn = xo + dt * d.fv[k];
-      if (stage == 1) d.fx0[k] = xo;
-      double xa = xn;
-      if (stage > 1 && i >= iL && i <= iR - 1) xa = w0 * d.fx0[k] + w1 * xn;
-      d.fxn[k] = xa;
-    }
-    if (stage > 1 && (i == iL || i == iR)) {
-      // CellGeomFromInterfacePos covers cells 1..ntrack-2 (1d.cpp:834), so the
-      // ghost cells next to the active range follow their faces too (split at
-      // the first / last active cell reads them)
-      double xoL = d.fx[k - 1] + dt * d.fv[k - 1];
-      double xoR = d.fx[k] + dt * d.fv[k];
-      if (i - 1 >= iL && i - 1 <= iR - 1) xoL = w0 * d.fx0[k - 1] + w1 * xoL;
-      if (i >= iL && i <= iR - 1) xoR = w0 * d.fx0[k] + w1 * xoR;
-      d.cx[k] = (xoR + xoL) / 2.;
-      d.cdx[k] = (xoR - xoL);
-    } else if (i >= iL + 1 && i <= iR - 1) {
-      cell = true;
-    }
-  }
   if (cell) {
-    xnL = d.fx[k - 1] + dt * d.fv[k - 1];
-    xnR = d.fx[k] + dt * d.fv[k];
     load_v<ND, NQ>(d, d.prim, k, p);
     Geo g = geo_of_g<ND>(d, j, k, geom);
     prim2cons<ND, NQ>(p, U, sweep_r<ND>(d, k, g), geom, G, d.P.synge);
@@ -925,8 +917,7 @@ GH_HD void body_update_g(const Dev& d, int j, int i, int stage, bool valid, cons
     for (int q = 0; q < NQ; ++q) U[q] *= g.dV;
     {
       double fa[NQ], fb[NQ];
-      load_v<ND, NQ>(d, d.fflux, k - 1, fa);
-      load_v<ND, NQ>(d, d.fflux, k, fb);
+      mv(fa, fb);
       for (int q = 0; q < NQ; ++q) U[q] += (fa[q] - fb[q]) * dt;
     }
     if (ND == 2) {   // net F1 flux: summed here, or read from body_f1sum's pass
@@ -967,8 +958,6 @@ GH_HD void body_update_g(const Dev& d, int j, int i, int stage, bool valid, cons
       load_v<ND, NQ>(d, d.U0, k, U0);
       double dV0 = d.dV0[k];
       for (int q = 0; q < NQ; ++q) U[q] = w0 * U0[q] * dV0 + w1 * U[q] * g2.dV;
-      double xaL = w0 * d.fx0[k - 1] + w1 * xnL;
-      double xaR = w0 * d.fx0[k] + w1 * xnR;
       cxn = (xaR + xaL) / 2.;
       cdxn = (xaR - xaL);
       Geo g3 = cell_geo<ND>(cxn, cdxn, d.ty[j], d.tdy[j], geom, trig_at_g<ND>(d, j, geom));
@@ -987,15 +976,70 @@ GH_HD void body_update_g(const Dev& d, int j, int i, int stage, bool valid, cons
     ncalls = 2;
   }
   if (!cell) return;
-  store_v<ND, NQ>(d, d.prim, k, p);
-  d.cx[k] = cxn;
-  d.cdx[k] = cdxn;
+  *cxo = cxn;
+  *cdxo = cdxn;
   GH_ATOMIC_ADD(cnt_at(d, CNT_C2P_CALLS), (unsigned long long)ncalls);
   if (st.iters) GH_ATOMIC_ADD(cnt_at(d, CNT_C2P_ITERS), (unsigned long long)st.iters);
   if (st.used) GH_ATOMIC_ADD(cnt_at(d, CNT_MLP), (unsigned long long)st.used);
   if (st.fail & 1) GH_ATOMIC_ADD(cnt_at(d, CNT_NOBRACKET), 1ull);
   if (st.fail & 2) GH_ATOMIC_ADD(cnt_at(d, CNT_MAXITER), 1ull);
   if (st.fail & 4) GH_ATOMIC_ADD(cnt_at(d, CNT_PHICAP), 1ull);
+}
+
+// GEO: the grid's geometry when fixed at compile time (2D grids have one;
+// -1: the track's, as 1D ensembles mix them)
+template <int ND, int NQ, int SV, class GuessT, int GEO = -1>
+GH_HD void body_update_g(const Dev& d, int j, int i, int stage, bool valid, const GuessT& guess) {
+  bool run = valid && active_track(d, j);
+  int nt = run ? d.ntrack[j] : 0;
+  run = run && i < nt;
+  int iL = d.ngst - 1, iR = nt - d.ngst;
+  int geom = GEO >= 0 ? GEO : run ? d.tgeom[j] : 0;
+  double dt = run ? d.tdt[j] : 0.;
+  double w0 = stage == 2 ? 3. / 4. : 1. / 3.;
+  double w1 = stage == 2 ? 1. / 4. : 2. / 3.;
+  long long k = run ? CI(d, j, i) : 0;
+  bool cell = false;
+  if (run) {
+    if (i <= nt - 2) {
+      double xo = d.fx[k];
+      double xn = xo + dt * d.fv[k];
+      if (stage == 1) d.fx0[k] = xo;
+      double xa = xn;
+      if (stage > 1 && i >= iL && i <= iR - 1) xa = w0 * d.fx0[k] + w1 * xn;
+      d.fxn[k] = xa;
+    }
+    if (stage > 1 && (i == iL || i == iR)) {
+      // CellGeomFromInterfacePos covers cells 1..ntrack-2 (1d.cpp:834), so the
+      // ghost cells next to the active range follow their faces too (split at
+      // the first / last active cell reads them)
+      double xoL = d.fx[k - 1] + dt * d.fv[k - 1];
+      double xoR = d.fx[k] + dt * d.fv[k];
+      if (i - 1 >= iL && i - 1 <= iR - 1) xoL = w0 * d.fx0[k - 1] + w1 * xoL;
+      if (i >= iL && i <= iR - 1) xoR = w0 * d.fx0[k] + w1 * xoR;
+      d.cx[k] = (xoR + xoL) / 2.;
+      d.cdx[k] = (xoR - xoL);
+    } else if (i >= iL + 1 && i <= iR - 1) {
+      cell = true;
+    }
+  }
+  double xnL = 0., xnR = 0., xaL = 0., xaR = 0., cxn, cdxn, p[NQ];
+  if (cell) {
+    xnL = d.fx[k - 1] + dt * d.fv[k - 1];
+    xnR = d.fx[k] + dt * d.fv[k];
+    if (stage > 1) {
+      xaL = w0 * d.fx0[k - 1] + w1 * xnL;
+      xaR = w0 * d.fx0[k] + w1 * xnR;
+    }
+  }
+  cell_advance<ND, NQ, SV>(d, j, i, k, geom, stage, dt, cell, xnL, xnR, xaL, xaR, [&](double* fa, double* fb) {
+    load_v<ND, NQ>(d, d.fflux, k - 1, fa);
+    load_v<ND, NQ>(d, d.fflux, k, fb);
+  }, guess, p, &cxn, &cdxn);
+  if (!cell) return;
+  store_v<ND, NQ>(d, d.prim, k, p);
+  d.cx[k] = cxn;
+  d.cdx[k] = cdxn;
 }
 
 // Grid::update + Cell::update + RK3 averages (1d.cpp:798-841, 2d.cpp:974-1036,
@@ -1011,6 +1055,191 @@ GH_HD void body_update(const Dev& d, int j, int i, int stage) {
   if (stage > 1) body_dt(d, j, i);         // the faces' dt candidates (prep with dt = false)
   if (d.solver == C2P_NEWTON) body_update_s<ND, NQ, C2P_NEWTON>(d, j, i, stage);
   else body_update_s<ND, NQ, C2P_BRENT>(d, j, i, stage);
+}
+
+// ---------------------------------------------------------------------------
+// The step of independent (1D) tracks in five passes, for gammahip_step:
+//   begin    regrid, then the ghost cells
+//   faces 1  resetShock, MV faces, detectShock, each tile's dt minimum
+//   stage 1  the tracks' dt, Grid::update, the next ghost cells
+//   stage 2  MV faces, dt candidates, Grid::update, the next ghost cells
+//   stage 3  MV faces, dt candidates, Grid::update, particles, time advance
+// in place of one launch per sweep (13 to 19 a step, of 4.5 us at least; a step
+// of a 64-cell track 93 -> 71 us, 4000 cells with particles 180 -> 128, 24
+// tracks 229 -> 135, 256 tracks 939 -> 770).  Small tracks are bound by the
+// latency of a cell's two root searches, the ensemble by FP64 issue (some 5900
+// vector instructions per wavefront and stage).  A stage reads the state
+// of cells its workgroup does not own, so it writes to a second set of planes
+// (primn, cxn, cdxn, fxn) that the driver swaps in.  Same arithmetic in the
+// same order as the separate sweeps.  Fluxes, signal speeds and face speeds go
+// to memory in the last stage only: nothing reads the others' outside the pass.
+
+// The stage passes write live cells only: slots past a track's end hold the
+// same values in both sets of planes (load, restore and regrid see to it), as
+// they would if the cells were advanced in place.
+GH_HD void mirror_slot(const Dev& d, long long k) {
+  for (int s = 0; s < d.nqs; ++s) d.primn[s * d.cs + k] = d.prim[s * d.cs + k];
+  d.cxn[k] = d.cx[k];
+  d.cdxn[k] = d.cdx[k];
+}
+
+// the part of stage passes' ghost copies a thread holds: an edge cell's new state
+template <int NQ>
+struct EdgeCell { double p[NQ], x, dx, f, dt, sd, ps; int sh; };
+
+// ghost cell i of track j in the new planes (body_ghost_mv on the stage's result)
+template <int NQ>
+GH_HD void s1_ghost(const Dev& d, int j, int nt, int i, const EdgeCell<NQ>& e) {
+  int iL = d.ngst - 1, iR = nt - d.ngst;
+  long long k = CI(d, j, i);
+  double p[NQ], x;
+  for (int q = 0; q < NQ; ++q) p[q] = e.p[q];
+  if (i <= iL) {
+    x = e.x - (iL - i + 1) * e.dx;
+    if (i <= iL - 1) d.fxn[k] = e.f - (iL - i + 1) * e.dx;
+    if (d.tbnd[j] == BND_BM) {
+      bm_profile(d.tbm + 4 * j, x, d.tt[j], d.P.gamma, &p[RHO], &p[UU1], &p[PPP]);
+      p[TR1] = 2.;
+    }
+  } else {
+    x = e.x + (i - iR + 1) * e.dx;
+    if (i <= nt - 2) d.fxn[k] = e.f + (i - iR) * e.dx;
+  }
+  store_v<1, NQ>(d, d.primn, k, p);
+  d.cxn[k] = x;
+  d.cdxn[k] = e.dx;
+  d.dtloc[k] = e.dt;
+  if (d.shock) { d.sd[k] = e.sd; d.pspec[k] = e.ps; d.shk[k] = e.sh; }
+}
+
+// a face as the two cells beside it use it
+template <int NQ>
+struct FaceOut { double v, lL, lR, xn, xa, fl[NQ], sd, ps; };
+
+// faces 1: face i of the track into o; own = false: a neighbour tile's face,
+// whose stores and counts are left to its owner
+template <int NQ, bool SHK>
+GH_HD void s1_face1(const Dev& d, int j, int nt, int i, bool own, FaceOut<NQ>& o) {
+  bool face = i >= 0 && i <= nt - 2;
+  long long k = CI(d, j, i);
+  double pL[NQ], pR[NQ], Sd = -1., ps = 0.;
+  if (face) {
+    Waves w;
+    face_flux<1, NQ>(d, j, i, nt, pL, pR, w, o.v, o.fl);
+    o.lL = w.lL;
+    o.lR = w.lR;
+    if (own) {
+      if (o.fl[0] != o.fl[0]) GH_ATOMIC_ADD(cnt_at(d, CNT_NANFLUX), 1ull);
+      d.fv[k] = o.v;
+      store_v<1, NQ>(d, d.fflux, k, o.fl);
+    }
+  }
+  if (SHK && own && i < d.nax) {        // resetShock, measureShock, detectShock
+    if (face) {
+      double p1 = -1.e300;
+      Sd = fmax(Sd, shock_sd<1, NQ>(pL, pR, 0, false, d.P.gamma, &p1, d.vpspec));
+      if (p1 > ps) ps = p1;
+    }
+    d.sd[k] = Sd;
+    d.pspec[k] = ps;
+    d.shk[k] = Sd > d.P.shock_thr ? 1 : 0;
+  }
+}
+// its dt candidate with the one carried over, which is reset (collect_dt)
+GH_HD double s1_dt1(const Dev& d, int j, int nt, int i, double vl, double lR, double vr, double lL) {
+  if (i >= nt) return 1.e15;
+  long long k = CI(d, j, i);
+  double v = d.dtloc[k];
+  if (i >= 1 && i <= nt - 2) {
+    double cand = dt_cand(d.cdx[k], vl, lR, vr, lL);
+    if (cand < 0) GH_ATOMIC_ADD(cnt_at(d, CNT_NEGDT), 1ull);
+    v = fmin(v, cand);
+  }
+  d.dtloc[k] = 1.e15;
+  return v;
+}
+
+// stage pass, face part: face i (0 <= i <= nt - 2) of the track into o.
+// Ghost cells' faces and values are left to s1_ghost where it follows.
+template <int NQ, bool SHK, int STAGE>
+GH_HD void s1_face(const Dev& d, int j, int nt, int i, double dt, bool own, FaceOut<NQ>& o) {
+  long long k = CI(d, j, i);
+  int iL = d.ngst - 1, iR = nt - d.ngst;
+  double xo = d.fx[k], x0 = STAGE > 1 ? d.fx0[k] : 0.;
+  if (STAGE == 1) {
+    o.v = d.fv[k];
+    load_v<1, NQ>(d, d.fflux, k, o.fl);
+    if (SHK) { o.sd = d.sd[k]; o.ps = d.pspec[k]; }
+  } else {
+    double pL[NQ], pR[NQ];
+    Waves w;
+    face_flux<1, NQ>(d, j, i, nt, pL, pR, w, o.v, o.fl);
+    o.lL = w.lL;
+    o.lR = w.lR;
+    if (own && o.fl[0] != o.fl[0]) GH_ATOMIC_ADD(cnt_at(d, CNT_NANFLUX), 1ull);
+    if (SHK && own) {
+      double p1 = -1.e300, Sd = shock_sd<1, NQ>(pL, pR, 0, false, d.P.gamma, &p1, d.vpspec);
+      o.sd = fmax(d.sd[k], Sd);
+      o.ps = d.pspec[k];
+      if (p1 > o.ps) o.ps = p1;
+    }
+  }
+  o.xn = xo + dt * o.v;
+  o.xa = o.xn;
+  if (STAGE > 1 && i >= iL && i <= iR - 1) {
+    double w0 = STAGE == 2 ? 3. / 4. : 1. / 3., w1 = STAGE == 2 ? 1. / 4. : 2. / 3.;
+    o.xa = w0 * x0 + w1 * o.xn;
+  }
+  if (!own) return;
+  if (STAGE == 1) d.fx0[k] = xo;
+  if (STAGE == 3 || (i > iL - 1 && i < iR)) d.fxn[k] = o.xa;
+  if (STAGE == 3) {
+    d.fv[k] = o.v;
+    d.flL[k] = o.lL;
+    d.flR[k] = o.lR;
+    store_v<1, NQ>(d, d.fflux, k, o.fl);
+  }
+  if (SHK && STAGE > 1 && (STAGE == 3 || (i > iL && i < iR))) { d.sd[k] = o.sd; d.pspec[k] = o.ps; }
+}
+// stage pass, cell part: cell i from its left face (values) and right face o.
+// Returns whether it is an active cell; its new state is then in e.
+template <int NQ, bool SHK, int SV, int STAGE, class LeftFlux>
+GH_HD bool s1_cell(const Dev& d, int j, int nt, int i, double dt, bool has, double vl, double lR, double xnL,
+                   double xaL, const LeftFlux& left, const FaceOut<NQ>& o, EdgeCell<NQ>& e) {
+  int iL = d.ngst - 1, iR = nt - d.ngst;
+  has = has && i < nt;
+  bool cell = has && i >= iL + 1 && i <= iR - 1;
+  long long k = has ? CI(d, j, i) : 0;
+  e.dt = 1.e15;
+  if (STAGE > 1 && has && i >= 1 && i <= nt - 2) {      // body_dt
+    double cand = dt_cand(d.cdx[k], vl, lR, o.v, o.lL);
+    if (cand < 0) GH_ATOMIC_ADD(cnt_at(d, CNT_NEGDT), 1ull);
+    if (STAGE == 3 || cell) d.dtloc[k] = e.dt = fmin(d.dtloc[k], cand);
+  }
+  double cxn = 0., cdxn = 0.;
+  cell_advance<1, NQ, SV>(d, j, i, k, has ? d.tgeom[j] : 0, STAGE, dt, cell, xnL, o.xn, xaL, o.xa,
+                          [&](double* fa, double* fb) {
+                            left(fa);
+                            for (int q = 0; q < NQ; ++q) fb[q] = o.fl[q];
+                          }, NoGuess{}, e.p, &cxn, &cdxn);
+  if (!has) return false;
+  if (!cell) {
+    if (STAGE < 3) return false;
+    load_v<1, NQ>(d, d.prim, k, e.p);                   // ghost cells of the last stage: kept, but for
+    cxn = d.cx[k];                                      // the positions of those between two faces
+    cdxn = d.cdx[k];
+    if (i == iL || i == iR) { cxn = (o.xa + xaL) / 2.; cdxn = o.xa - xaL; }
+  }
+  if (STAGE == 3 && NQ == 10 && d.sync)
+    inject<1, NQ>(e.p, SHK && d.shk[k] != 0, !SHK ? 0. : i <= nt - 2 ? o.ps : d.pspec[k], d.P);
+  store_v<1, NQ>(d, d.primn, k, e.p);
+  d.cxn[k] = cxn;
+  d.cdxn[k] = cdxn;
+  e.x = cxn;
+  e.dx = cdxn;
+  e.f = o.xa;
+  if (STAGE < 3 && SHK) { e.sd = o.sd; e.ps = o.ps; e.sh = d.shk[k]; }
+  return cell;
 }
 
 // ---------------------------------------------------------------------------
@@ -2027,11 +2256,10 @@ __device__ bool wg_screen(const Dev& d, int j, bool bm, int* red, int* i0, int* 
   return *i1 >= 0;
 }
 template <int ND, int NQ>
-__global__ void __launch_bounds__(RGB) k_regrid(Dev d) {
+__device__ void wg_regrid(const Dev& d, int j) {
   __shared__ int red[RGB];
   __shared__ double rv[RGB];
   __shared__ int s_act;
-  int j = blockIdx.x;
   if (!active_track(d, j) || d.trg[j] == RG_NONE) return;
   bool bm = d.trg[j] == RG_BM1D;
   long long b = CI(d, j, 0);
@@ -2042,6 +2270,7 @@ __global__ void __launch_bounds__(RGB) k_regrid(Dev d) {
   if (d.circ) wg_victims<ND, NQ>(d, j, rv, red, &is, &ib);
   RgStop stop = rg_stop_init(d, j, iS, tl);
   int last_mod = -1;                       // the last cell a split or merge wrote
+  int ntmax = d.ntrack[j];                 // the longest the track has been in this pass
   for (;;) {
     int nt = d.ntrack[j];
     int last = nt - d.ngst - 1;
@@ -2080,13 +2309,14 @@ __global__ void __launch_bounds__(RGB) k_regrid(Dev d) {
     i += first;
     int act = s_act, delta = 0;
     __syncthreads();
-    // is, ib and i are the same on every lane: a clash returns the whole workgroup
+    if (act == 1 && nt + 1 > ntmax) ntmax = nt + 1;
+    // is, ib and i are the same on every lane: a clash ends the loop on all of them
     if (act == 1) {
       int isplit = i;
       if (d.circ) {
         if (is < 0 || is == i) {
           if (threadIdx.x == 0) GH_ATOMIC_ADD(cnt_at(d, CNT_RGCLASH), 1ull);
-          return;
+          break;
         }
         wg_merge<ND, NQ>(d, j, b, is, &s_act);
         if (i > is) isplit--;
@@ -2097,7 +2327,7 @@ __global__ void __launch_bounds__(RGB) k_regrid(Dev d) {
     } else {
       if (d.circ && (ib < 0 || ib == i)) {
         if (threadIdx.x == 0) GH_ATOMIC_ADD(cnt_at(d, CNT_RGCLASH), 1ull);
-        return;
+        break;
       }
       wg_merge<ND, NQ>(d, j, b, i, &s_act);
       if (d.circ) wg_split<ND, NQ>(d, j, b, ib > i ? ib - 1 : ib);
@@ -2107,6 +2337,95 @@ __global__ void __launch_bounds__(RGB) k_regrid(Dev d) {
     if (bm) iS = !d.circ && rg_shock_shifts(iS, delta, last_mod) ? iS + delta : wg_shock_index(d, j, red);
     if (d.circ) wg_victims<ND, NQ>(d, j, rv, red, &is, &ib);
     ++i;
+  }
+  if (ND == 1) {
+    __syncthreads();
+    for (int m = d.ntrack[j] + (int)threadIdx.x; m < ntmax; m += RGB) mirror_slot(d, b + m);
+  }
+}
+template <int ND, int NQ>
+__global__ void __launch_bounds__(RGB) k_regrid(Dev d) { wg_regrid<ND, NQ>(d, (int)blockIdx.x); }
+
+// ---- the five passes of a 1D step (see s1_face1) ----
+// begin: one workgroup per track; RG: some track has a regrid rule
+template <int NQ, bool RG>
+__global__ void __launch_bounds__(RG ? RGB : 64) k1_begin(Dev d) {
+  int j = (int)blockIdx.x;
+  if (RG) {
+    wg_regrid<1, NQ>(d, j);
+    __syncthreads();
+  }
+  if ((int)threadIdx.x < 2 * d.ngst) body_ghost_mv<1, NQ>(d, j, (int)threadIdx.x);
+}
+template <int NQ, bool SHK>
+__global__ void __launch_bounds__(S1B) k1_faces(Dev d) {
+  __shared__ double sv[S1B], sl[S1B], sm[S1B / 64];
+  int j = (int)blockIdx.y, t = (int)threadIdx.x, i = (int)blockIdx.x * S1C + t - 1;
+  int nt = d.ntrack[j];
+  FaceOut<NQ> o;
+  o.v = 0.; o.lL = 0.; o.lR = 0.;
+  if ((int)blockIdx.x * S1C < nt || SHK) s1_face1<NQ, SHK>(d, j, nt, i, t > 0, o);
+  if ((int)blockIdx.x * S1C >= nt) return;
+  sv[t] = o.v;
+  sl[t] = o.lR;
+  __syncthreads();
+  double m = t > 0 ? s1_dt1(d, j, nt, i, sv[t - 1], sl[t - 1], o.v, o.lL) : 1.e15;
+  for (int s = 32; s > 0; s >>= 1) m = fmin(m, __shfl_xor(m, s, 64));
+  if ((t & 63) == 0) sm[t >> 6] = m;
+  __syncthreads();
+  if (t == 0) {
+    for (int q = 1; q < S1B / 64; ++q) m = fmin(m, sm[q]);
+    d.tpart[(long long)j * d.s1ch + blockIdx.x] = m;
+  }
+}
+template <int NQ, bool SHK, int SV, int STAGE>
+__global__ void __launch_bounds__(S1B) k1_stage(Dev d) {
+  constexpr int NS = NQ - 1;
+  __shared__ double sv[S1B], sl[S1B], sx[S1B], sa[S1B], sf[NS][S1B];
+  int j = (int)blockIdx.y, t = (int)threadIdx.x, i = (int)blockIdx.x * S1C + t - 1;
+  int nt = d.ntrack[j];
+  if ((int)blockIdx.x * S1C >= nt) return;
+  double dt;
+  if (STAGE == 1) {
+    // the track's minimum over its tiles, by every wavefront for itself (a
+    // minimum does not depend on the order it is taken in)
+    double m = 1.e15;
+    int n = (nt + S1C - 1) / S1C;
+    for (int q = t & 63; q < n; q += 64) m = fmin(m, d.tpart[(long long)j * d.s1ch + q]);
+    for (int s = 32; s > 0; s >>= 1) m = fmin(m, __shfl_xor(m, s, 64));
+    dt = d.P.cfl * m;
+    if (blockIdx.x == 0 && t == 0) { d.tmin[j] = m; d.tdt[j] = dt; }
+  } else {
+    dt = d.tdt[j];
+  }
+  FaceOut<NQ> o;
+  o.v = 0.; o.lL = 0.; o.lR = 0.; o.xn = 0.; o.xa = 0.; o.sd = -1.; o.ps = 0.;
+  for (int q = 0; q < NQ; ++q) o.fl[q] = 0.;
+  if (i >= 0 && i <= nt - 2) s1_face<NQ, SHK, STAGE>(d, j, nt, i, dt, t > 0, o);
+  sv[t] = o.v; sl[t] = o.lR; sx[t] = o.xn; sa[t] = o.xa;
+  for (int q = 0; q < NQ; ++q)
+    if (q != 3) sf[sq<1>(q)][t] = o.fl[q];
+  __syncthreads();
+  int tl = t > 0 ? t - 1 : 0;
+  EdgeCell<NQ> e;
+  bool cell = s1_cell<NQ, SHK, SV, STAGE>(d, j, nt, i, dt, t > 0, sv[tl], sl[tl], sx[tl], sa[tl], [&](double* fa) {
+    for (int q = 0; q < NQ; ++q) fa[q] = q == 3 ? 0. : sf[sq<1>(q)][tl];
+  }, o, e);
+  if (STAGE < 3) {
+    if (cell && i == nt - d.ngst - 1) {
+      for (int g = 0; g < d.ngst; ++g) s1_ghost<NQ>(d, j, nt, nt - d.ngst + g, e);
+    }
+    if (blockIdx.x == 0 && t < 64) {          // cells -1 .. 62: the first active cell and the left ghost cells
+      EdgeCell<NQ> f;
+      int src = d.ngst + 1;
+      for (int q = 0; q < NQ; ++q) f.p[q] = __shfl(e.p[q], src, 64);
+      f.x = __shfl(e.x, src, 64); f.dx = __shfl(e.dx, src, 64); f.f = __shfl(e.f, src, 64);
+      f.dt = __shfl(e.dt, src, 64);
+      if (SHK) { f.sd = __shfl(e.sd, src, 64); f.ps = __shfl(e.ps, src, 64); f.sh = __shfl(e.sh, src, 64); }
+      if (i >= 0 && i < d.ngst) s1_ghost<NQ>(d, j, nt, i, f);
+    }
+  } else if (blockIdx.x == 0 && t == 0) {
+    d.tt[j] += dt;
   }
 }
 }  // namespace
@@ -2481,6 +2800,7 @@ struct gammahip_ctx {
                            // bit 1: MV gradients recomputed in the F1 passes (Dev::gmvre);
                            // bit 2: F1 face pass one thread per owner cell (k_f1own)
   int ncu = 256;           // compute units of the device
+  bool user_hooks = false; // some track has user kinematics or boundaries
 #ifndef GH_EMU
   hipStream_t stream = nullptr;
   // event pairs of timed launches, read back when the times are asked for
@@ -2545,6 +2865,23 @@ int d2h(gammahip_ctx* c, void* dst, const void* src, size_t bytes) {
   HIPCHK(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
   return 0;
 #endif
+}
+
+// 1D: the stage passes' second planes take the values of the first (which hold
+// the state just loaded or restored)
+int mirror_state(gammahip_ctx* c) {
+  Dev& d = c->d;
+  if (d.nd != 1) return 0;
+  std::pair<double*, double*> pl[3] = {{d.primn, d.prim}, {d.cxn, d.cx}, {d.cdxn, d.cdx}};
+  for (int q = 0; q < 3; ++q) {
+    size_t bytes = sizeof(double) * (size_t)d.cs * (q == 0 ? d.nqs : 1);
+#ifdef GH_EMU
+    memcpy(pl[q].first, pl[q].second, bytes);
+#else
+    HIPCHK(hipMemcpyAsync(pl[q].first, pl[q].second, bytes, hipMemcpyDeviceToDevice, c->stream));
+#endif
+  }
+  return 0;
 }
 
 // ---- launches ----
@@ -2909,7 +3246,11 @@ struct Pipe {
     L2(c, body_rg_init, d.nj, 1);
     if (d.rg_mode & (1 << RG_BM1D)) L2(c, body_rg_shockpos, d.nj, d.nax);
     L2(c, (body_rg_screen<ND, NQ>), d.nj, d.nax);
-    for (int j = 0; j < d.nj; ++j) body_rg_apply<ND, NQ>(d, j, 0);
+    for (int j = 0; j < d.nj; ++j) {
+      body_rg_apply<ND, NQ>(d, j, 0);
+      if (ND == 1)
+        for (int i = d.ntrack[j]; i < d.nax; ++i) mirror_slot(d, CI(d, j, i));
+    }
 #else
     hipLaunchKernelGGL((k_regrid<ND, NQ>), dim3(d.nj), dim3(RGB), 0, c->stream, d);
 #endif
@@ -2932,8 +3273,82 @@ struct Pipe {
     ghosts(c); prep(c, false); update(c, 2);
     ghosts(c); prep(c, false); update(c, 3);
   }
+  // the 1D step in five passes; general otherwise: packed launches, the learned
+  // start, Euler steps, event timing of the separate passes, and user hooks
+  // that read the track's time while a stage runs
+  static bool fused1(const gammahip_ctx* c) {
+    const Dev& d = c->d;
+    return ND == 1 && !d.packed && !d.mw && !d.euler && !d.ucell && !c->timing && !c->user_hooks;
+  }
+  template <bool SHK>
+  static void step1(gammahip_ctx* c) {
+    Dev& d = c->d;
+    auto swap = [&]() {
+      std::swap(d.prim, d.primn); std::swap(d.cx, d.cxn); std::swap(d.cdx, d.cdxn); std::swap(d.fx, d.fxn);
+    };
+#ifdef GH_EMU
+    regrid(c);
+    L2(c, (body_ghost_mv<ND, NQ>), d.nj, 2 * d.ngst);
+    std::vector<FaceOut<NQ>> F(d.nax);
+    for (int j = 0; j < d.nj; ++j) {
+      int nt = d.ntrack[j];
+      for (int i = 0; i < d.nax; ++i) s1_face1<NQ, SHK>(d, j, nt, i, true, F[i]);
+      double m = 1.e15;
+      for (int i = 0; i < nt; ++i)
+        m = fmin(m, s1_dt1(d, j, nt, i, i ? F[i - 1].v : 0., i ? F[i - 1].lR : 0., F[i].v, F[i].lL));
+      d.tmin[j] = m;
+      d.tdt[j] = d.P.cfl * m;
+    }
+    auto stage = [&](auto st, auto sv) {
+      constexpr int ST = decltype(st)::value, SV = decltype(sv)::value;
+      for (int j = 0; j < d.nj; ++j) {
+        int nt = d.ntrack[j];
+        double dt = d.tdt[j];
+        for (int i = 0; i <= nt - 2; ++i) s1_face<NQ, SHK, ST>(d, j, nt, i, dt, true, F[i]);
+        for (int i = 0; i < nt; ++i) {
+          const FaceOut<NQ>& L = F[i ? i - 1 : 0];
+          EdgeCell<NQ> e;
+          bool cell = s1_cell<NQ, SHK, SV, ST>(d, j, nt, i, dt, true, L.v, L.lR, L.xn, L.xa, [&](double* fa) {
+            for (int q = 0; q < NQ; ++q) fa[q] = L.fl[q];
+          }, F[i], e);
+          if (ST == 3 || !cell) continue;
+          for (int g = 0; g < d.ngst; ++g) {
+            if (i == d.ngst) s1_ghost<NQ>(d, j, nt, g, e);
+            if (i == nt - d.ngst - 1) s1_ghost<NQ>(d, j, nt, nt - d.ngst + g, e);
+          }
+        }
+        if (ST == 3) d.tt[j] += dt;
+      }
+      swap();
+    };
+#else
+    dim3 tiles(d.s1ch, d.nj);
+    if (d.rg_mode) hipLaunchKernelGGL((k1_begin<NQ, true>), dim3(d.nj), dim3(RGB), 0, c->stream, d);
+    else hipLaunchKernelGGL((k1_begin<NQ, false>), dim3(d.nj), dim3(64), 0, c->stream, d);
+    hipLaunchKernelGGL((k1_faces<NQ, SHK>), tiles, dim3(S1B), 0, c->stream, d);
+    auto stage = [&](auto st, auto sv) {
+      constexpr int ST = decltype(st)::value, SV = decltype(sv)::value;
+      hipLaunchKernelGGL((k1_stage<NQ, SHK, SV, ST>), tiles, dim3(S1B), 0, c->stream, d);
+      swap();
+    };
+#endif
+    auto all = [&](auto sv) {
+      stage(std::integral_constant<int, 1>{}, sv);
+      stage(std::integral_constant<int, 2>{}, sv);
+      stage(std::integral_constant<int, 3>{}, sv);
+    };
+    if (d.solver == C2P_NEWTON) all(std::integral_constant<int, C2P_NEWTON>{});
+    else all(std::integral_constant<int, C2P_BRENT>{});
+  }
   // one iteration of Simu::run (simu.cpp:47-77)
   static void step(gammahip_ctx* c) {
+    if constexpr (ND == 1) {
+      if (fused1(c)) {
+        if (c->d.shock) step1<true>(c);
+        else step1<false>(c);
+        return;
+      }
+    }
     regrid(c);
     apply(c, GAMMAHIP_RESET_SHOCK);
     ghosts(c, true);          // track lengths settle here: rebuild the tile list
@@ -3069,13 +3484,15 @@ int gammahip_create(const gammahip_config* cfg, gammahip_ctx** out) {
   e |= dalloc(c, &d.ty, nj); e |= dalloc(c, &d.tdy, nj); e |= dalloc(c, &d.tdt, nj);
   e |= dalloc(c, &d.tt, nj); e |= dalloc(c, &d.tmin, nj);
   d.dtch = (d.nax + DT_CH - 1) / DT_CH;
-  e |= dalloc(c, &d.tpart, nj * (size_t)d.dtch);
+  d.s1ch = (d.nax + S1C - 1) / S1C;
+  e |= dalloc(c, &d.tpart, nj * (size_t)std::max(d.dtch, d.s1ch));
   e |= dalloc(c, &d.prim, nqs * cs); e |= dalloc(c, &d.cx, cs); e |= dalloc(c, &d.cdx, cs);
   e |= dalloc(c, &d.dtloc, cs); e |= dalloc(c, &d.U0, nqs * cs); e |= dalloc(c, &d.dV0, cs);
   e |= dalloc(c, &d.fx, cs); e |= dalloc(c, &d.fxn, cs); e |= dalloc(c, &d.fx0, cs);
   e |= dalloc(c, &d.fv, cs); e |= dalloc(c, &d.flL, cs); e |= dalloc(c, &d.flR, cs);
   e |= dalloc(c, &d.fflux, nqs * cs);
   e |= dalloc(c, &d.cnt, (size_t)CNT_N * CNT_PARTS); e |= dalloc(c, &d.nsplit, nj); e |= dalloc(c, &d.nmerge, nj);
+  if (d.nd == 1) { e |= dalloc(c, &d.primn, nqs * cs); e |= dalloc(c, &d.cxn, cs); e |= dalloc(c, &d.cdxn, cs); }
   if (d.nd == 2) {
     e |= dalloc(c, &d.gmv, nqs * cs); e |= dalloc(c, &d.gf1, nqs * cs); e |= dalloc(c, &d.gf1n, nqs * cs);
     e |= dalloc(c, &d.nbdj, cs); e |= dalloc(c, &d.nbdlo, cs); e |= dalloc(c, &d.nbdcnt, cs);
@@ -3120,6 +3537,7 @@ int gammahip_load(gammahip_ctx* c, const double* x, const double* dx, const doub
   const gammahip_config& cf = c->cfg;
   int nj = d.nj, nax = d.nax, ng = d.ngst, nm = cf.ncell_mv, na = cf.ntracks_active;
   size_t cs = d.cs;
+  c->user_hooks = false;
   // host images of the initial state (Cinit + mpi_distribute, 1d.cpp:956-969, 2d.cpp:1175-1195)
   std::vector<int> ntrack(nj, nm + 2 * ng), tgeom(nj), tkin(nj), tbnd(nj), trg(nj, RG_NONE);
   std::vector<double> tvin(nj), tvout(nj), tbm(4 * nj), ty(nj), tdy(nj), tt(nj, t0);
@@ -3137,6 +3555,7 @@ int gammahip_load(gammahip_ctx* c, const double* x, const double* dx, const doub
     trg[j] = h.rg_mode >= 0 ? h.rg_mode : cf.rg_mode;
     d.rg_mode |= trg[j] != RG_NONE ? (1 << trg[j]) : 0;
     tgeom[j] = cf.geom >= 0 ? cf.geom : h.geom;
+    c->user_hooks |= h.kin_mode == KIN_USER || h.bnd_mode == BND_USER;
     tkin[j] = h.kin_mode; tvin[j] = h.v_in; tvout[j] = h.v_out; tbnd[j] = h.bnd_mode;
     for (int q = 0; q < 4; ++q) tbm[4 * j + q] = h.bm[q];
     ty[j] = cf.nd == 2 ? y[a] : 0.;
@@ -3212,7 +3631,7 @@ int gammahip_load(gammahip_ctx* c, const double* x, const double* dx, const doub
   e |= h2d(c, d.cdx, hdx.data(), sizeof(double) * cs);
   e |= h2d(c, d.fx, hfx.data(), sizeof(double) * cs);
   e |= h2d(c, d.dtloc, hdt.data(), sizeof(double) * cs);
-  if (e) return -1;
+  if (e || mirror_state(c)) return -1;
   if (d.shock) {
     std::vector<double> m1(cs, -1.);
     e |= h2d(c, d.sd, m1.data(), sizeof(double) * cs);
@@ -3488,6 +3907,7 @@ int gammahip_state_restore(gammahip_ctx* c, const void* buf, unsigned long long 
     if (h2d(c, s.p, o, s.bytes)) return -1;
     o += s.pad;
   }
+  if (mirror_state(c)) return -1;
   // the restored track lengths replace the loaded ones: the packed launch's
   // tile list must cover them before the next step's regrid screens the cells
   build_tiles(c);
