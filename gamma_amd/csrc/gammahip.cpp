@@ -1670,14 +1670,15 @@ GH_HD void body_advance_time(const Dev& d, int j, int i) {
 // as varying per lane: per-track values would then be loaded per lane and
 // same-address atomics (the shock-index maximum) issued per lane instead of
 // once per wavefront (0.025 -> 0.7 ms per launch on the 1D ensemble).
-__device__ __forceinline__ void tile_of(int remap, int& j, int& i) {
+// y0: rows of the grid in front of the tiles, which do something else
+__device__ __forceinline__ void tile_of(int remap, int& j, int& i, int y0 = 0) {
   if (remap == 2) {
-    j = __builtin_amdgcn_readfirstlane((int)blockIdx.y * (int)(blockDim.x >> 6) + (int)(threadIdx.x >> 6));
+    j = __builtin_amdgcn_readfirstlane(((int)blockIdx.y - y0) * (int)(blockDim.x >> 6) + (int)(threadIdx.x >> 6));
     i = (int)blockIdx.x * 64 + (int)(threadIdx.x & 63);
     return;
   }
-  int gx = gridDim.x, gy = gridDim.y;
-  int L = blockIdx.x + gx * blockIdx.y;
+  int gx = gridDim.x, gy = (int)gridDim.y - y0;
+  int L = blockIdx.x + gx * ((int)blockIdx.y - y0);
   if (remap) {
     // XCD x runs blocks x, x+8, x+16, ...: n_x = N/8 + (x < N%8) of them.  Give
     // it the logical range [x*(N/8) + min(x, N%8), +n_x): a bijection on [0, N).
@@ -1832,6 +1833,74 @@ template <bool PK, int ND, int NQ, bool SHK>
 __global__ void __launch_bounds__(KB, (SHK || NQ > 6) ? 1 : 5) k_faces(Dev d, int ni, int remap) {
   GH_TILE_LOOP(PK, if (i < ni && j < d.nj) body_faces_s<ND, NQ, SHK>(d, j, i))
 }
+// MV faces and F1 neighbour search of a 2D grid in one launch, in track-group
+// order: of 16 workgroups the first 8 (one per XCD) take face tiles, the others
+// the search on the same tiles.  Neither reads what the other writes; the faces
+// are bound by FP64 issue (73 % of their cycles), the search by the latency of
+// its chains of loads, so on grids that leave the chip part idle they run side
+// by side (FACES_NB_LIVE): 96 x 33 cells 233 -> 218 us a step, 512 x 129
+// 270 -> 265, 48 uneven tracks 483 -> 457.
+template <int NQ, bool SHK>
+__global__ void __launch_bounds__(KB, (SHK || NQ > 6) ? 1 : 5) k_faces_nb(Dev d, int gx, int n) {
+  int b = (int)blockIdx.x, f = (b >> 4) * 8 + (b & 7);
+  if (f >= n) return;
+  int g = f / gx;
+  int j = __builtin_amdgcn_readfirstlane(g * (int)(blockDim.x >> 6) + (int)(threadIdx.x >> 6));
+  int i = (f - g * gx) * 64 + (int)(threadIdx.x & 63);
+  bool in = i < d.nax && j < d.nj;
+  if (b & 8) body_nb_lanes(d, j, i, in);
+  else if (in) body_faces_s<2, NQ, SHK>(d, j, i);
+}
+// exclusive prefix sum of upper-neighbour counts along each track (F1 face slots)
+// inclusive prefix sum of one value per thread over the workgroup: shuffles
+// within each wavefront, the wavefront totals through LDS; *total = the sum
+// over the workgroup
+__device__ int wg_scan_incl(int v, int* wsum, int* total) {
+  int lane = (int)(threadIdx.x & 63), w = (int)(threadIdx.x >> 6);
+  for (int o = 1; o < 64; o <<= 1) {
+    int t = __shfl_up(v, o, 64);
+    if (lane >= o) v += t;
+  }
+  if (lane == 63) wsum[w] = v;
+  __syncthreads();
+  int add = 0, tot = 0;
+  for (int q = 0; q < (int)(blockDim.x >> 6); ++q) {
+    if (q < w) add += wsum[q];
+    tot += wsum[q];
+  }
+  __syncthreads();
+  *total = tot;
+  return v + add;
+}
+// Per track: exclusive scans of the F1 face counts (slot offsets, owner of
+// each slot, the track's total) and of the fresh-source counts (down-slot
+// offsets), a workgroup's threads at a time; the next chunk's counts are loaded while the
+// current chunk is scanned.
+__device__ void wg_f1_scan(const Dev& d, int j) {
+  __shared__ int wsum[KB / 64];
+  int B = (int)blockDim.x;
+  int nt = d.ntrack[j];
+  const int* cnt = d.nbucnt;
+  int base = 0;
+  int vnext = (int)threadIdx.x < nt ? cnt[CI(d, j, threadIdx.x)] : 0;
+  for (int i0 = 0; i0 < nt; i0 += B) {
+    int i = i0 + (int)threadIdx.x;
+    int v = vnext < 0 ? 0 : vnext;
+    vnext = i + B < nt ? cnt[CI(d, j, i + B)] : 0;
+    int tot;
+    int off = base + wg_scan_incl(v, wsum, &tot) - v;
+    if (i < nt) {
+      d.f1off[CI(d, j, i)] = off;
+      for (int n = 0; n < v && off + n < d.fcap; ++n) d.f1own[(long long)j * d.fcap + off + n] = i;
+    }
+    base += tot;
+  }
+  if (threadIdx.x == 0) {
+    d.f1tot[j] = base;
+    if (base > d.fcap) atomicAdd(cnt_at(d, CNT_F1OVF), 1ull);
+  }
+}
+__global__ void __launch_bounds__(KB) k_f1_scan(Dev d) { wg_f1_scan(d, (int)blockIdx.x); }
 // cell pass with the gradient cache in LDS: thread t's entry m at
 // cache[m * blockDim + t] (consecutive lanes, consecutive banks); the launch
 // passes blockDim * f1_kc * NQ doubles of dynamic LDS.  The pass waits on
@@ -1840,10 +1909,24 @@ __global__ void __launch_bounds__(KB, (SHK || NQ > 6) ? 1 : 5) k_faces(Dev d, in
 // (0.336 against 0.363 ms on the 2048^2 grid)
 template <bool PK, int NQ, int GEO>
 __global__ void __launch_bounds__(KB) __attribute__((amdgpu_waves_per_eu(1, 3)))
-k_f1grad(Dev d, int ni, int remap) {
+k_f1grad(Dev d, int ni, int remap, int y0) {
   extern __shared__ double f1cache[];
   double* cache = f1cache + threadIdx.x;
-  GH_TILE_LOOP(PK, if (i < ni && j < d.nj) body_f1grad_c<NQ, GEO>(d, j, i, cache, (int)blockDim.x))
+  if constexpr (!PK) {
+    // the plain launch scans the F1 face slots in y0 rows of workgroups, one
+    // per track, in front: no gradient reads a slot (a launch less per stage,
+    // 2 to 4 % of a step on grids to 512 x 512, 0.5 % on the largest)
+    if ((int)blockIdx.y < y0) {
+      int j = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+      if (j < d.nj) wg_f1_scan(d, j);
+      return;
+    }
+    int i, j;
+    tile_of(remap, j, i, y0);
+    if (i < ni && j < d.nj) body_f1grad_c<NQ, GEO>(d, j, i, cache, (int)blockDim.x);
+  } else {
+    GH_TILE_LOOP(true, if (i < ni && j < d.nj) body_f1grad_c<NQ, GEO>(d, j, i, cache, (int)blockDim.x))
+  }
 }
 // Neighbour search and transverse gradient in one pass (launch option FUSE
 // bit 0): a cell's gradient (2d.cpp:366-430) reads only its own neighbour
@@ -1994,55 +2077,6 @@ __global__ void __launch_bounds__(KB) k_dt_finish(Dev d) {
     __syncthreads();
   }
   for (int j = threadIdx.x; j < d.nj; j += KB) d.tdt[j] = d.P.cfl * (d.nd == 2 ? sm[0] : d.tmin[j]);
-}
-// exclusive prefix sum of upper-neighbour counts along each track (F1 face slots)
-// inclusive prefix sum of one value per thread over the workgroup: shuffles
-// within each wavefront, the wavefront totals through LDS; *total = the sum
-// over the workgroup
-__device__ int wg_scan_incl(int v, int* wsum, int* total) {
-  int lane = (int)(threadIdx.x & 63), w = (int)(threadIdx.x >> 6);
-  for (int o = 1; o < 64; o <<= 1) {
-    int t = __shfl_up(v, o, 64);
-    if (lane >= o) v += t;
-  }
-  if (lane == 63) wsum[w] = v;
-  __syncthreads();
-  int add = 0, tot = 0;
-  for (int q = 0; q < KB / 64; ++q) {
-    if (q < w) add += wsum[q];
-    tot += wsum[q];
-  }
-  __syncthreads();
-  *total = tot;
-  return v + add;
-}
-// Per track: exclusive scans of the F1 face counts (slot offsets, owner of
-// each slot, the track's total) and of the fresh-source counts (down-slot
-// offsets), KB cells at a time; the next chunk's counts are loaded while the
-// current chunk is scanned.
-__global__ void __launch_bounds__(KB) k_f1_scan(Dev d) {
-  __shared__ int wsum[KB / 64];
-  int j = blockIdx.x;
-  int nt = d.ntrack[j];
-  const int* cnt = d.nbucnt;
-  int base = 0;
-  int vnext = (int)threadIdx.x < nt ? cnt[CI(d, j, threadIdx.x)] : 0;
-  for (int i0 = 0; i0 < nt; i0 += KB) {
-    int i = i0 + (int)threadIdx.x;
-    int v = vnext < 0 ? 0 : vnext;
-    vnext = i + KB < nt ? cnt[CI(d, j, i + KB)] : 0;
-    int tot;
-    int off = base + wg_scan_incl(v, wsum, &tot) - v;
-    if (i < nt) {
-      d.f1off[CI(d, j, i)] = off;
-      for (int n = 0; n < v && off + n < d.fcap; ++n) d.f1own[(long long)j * d.fcap + off + n] = i;
-    }
-    base += tot;
-  }
-  if (threadIdx.x == 0) {
-    d.f1tot[j] = base;
-    if (base > d.fcap) atomicAdd(cnt_at(d, CNT_F1OVF), 1ull);
-  }
 }
 // The applyRegrid loop of one track on one workgroup, in the sequential
 // order.  The rule is evaluated for RGB cells at once (nothing it reads
@@ -2774,6 +2808,17 @@ struct KTimer {
   long long n;
 };
 
+// Rules of the 2D launches, in wavefronts of 64 live cells (counted at load).
+// Faces and neighbour search share a launch up to 3072 (three per SIMD, what
+// the gradient pass holds): 512 x 256 cells 349 -> 344 us a step, 512 x 512
+// 473 -> 475, 2048 x 512 1190 -> 1228, where each already fills the chip and
+// the two evict each other's lines.  Per-cell kernels take workgroups of one
+// wavefront up to 1024 (one per SIMD), which spreads them over the most CUs:
+// 96 x 33 cells 218 -> 201 us, 256 x 160 237 -> 232, 48 uneven tracks
+// 457 -> 418; 512 x 129 (1197) 265 -> 277, its two adjacent tracks in one
+// workgroup reading the same lines.
+constexpr long long FACES_NB_LIVE = 3072, BLOCK64_LIVE = 1024;
+
 struct gammahip_ctx {
   gammahip_config cfg;
   Dev d;
@@ -2790,6 +2835,8 @@ struct gammahip_ctx {
   // 2 % faster); the XCD bands help the uniform grid a little more but cost
   // the uneven ones up to 2x
   int block = 128;         // threads per workgroup of the per-cell kernels (64..256)
+  bool block_auto = true;  // block follows BLOCK64_LIVE until the option sets it (2D)
+  long long live = 0;      // wavefronts of 64 live cells at load
   int remap = 2;           // tile order: 0 hardware, 1 XCD bands, 2 track groups
   int use_graph = 0;       // replay steps from a captured hipGraph
   int persist = 0;         // packed launch: at most this many persistent workgroups per CU (0: off),
@@ -3041,18 +3088,31 @@ struct Pipe {
   // the next step's collect_dt), which has the cell's faces at hand
   static void prep(gammahip_ctx* c, bool dt = true) {
     Dev& d = c->d;
+    // FUSE bit 0: the neighbour search runs inside the gradient pass below
+    // (the slot scan after it needs only the lists)
+    bool nbgrad = ND == 2 && (c->fuse & 1) && !d.pc && !c->f1cell;
+    bool faces_nb = ND == 2 && !d.packed && !nbgrad && c->live <= FACES_NB_LIVE;
+#ifdef GH_EMU
+    nbgrad = faces_nb = false;     // the CPU build runs the bodies as separate sweeps
+#endif
     tbeg(c, 1);
-    if (d.shock) L2P(c, (body_faces<ND, NQ>), k_faces, (, ND, NQ, true), d.nj, d.nax);
-    else L2P(c, (body_faces<ND, NQ>), k_faces, (, ND, NQ, false), d.nj, d.nax);
+    if (faces_nb) {
+#ifndef GH_EMU
+      if constexpr (ND == 2) {
+        int gx = (d.nax + 63) / 64, W = c->block / 64, n = gx * ((d.nj + W - 1) / W);
+        dim3 g((unsigned)((n + 7) / 8 * 16));
+        if (d.shock) hipLaunchKernelGGL((k_faces_nb<NQ, true>), g, dim3(c->block), 0, c->stream, d, gx, n);
+        else hipLaunchKernelGGL((k_faces_nb<NQ, false>), g, dim3(c->block), 0, c->stream, d, gx, n);
+      }
+#endif
+    } else if (d.shock) {
+      L2P(c, (body_faces<ND, NQ>), k_faces, (, ND, NQ, true), d.nj, d.nax);
+    } else {
+      L2P(c, (body_faces<ND, NQ>), k_faces, (, ND, NQ, false), d.nj, d.nax);
+    }
     tend(c, 1);
     if (dt) L2P(c, body_dt, k_dt, (), d.nj, d.nax);
     if (ND == 2) {
-      // FUSE bit 0: the neighbour search runs inside the gradient pass below
-      // (the slot scan after it needs only the lists)
-      bool nbgrad = (c->fuse & 1) && !d.pc && !c->f1cell;
-#ifdef GH_EMU
-      nbgrad = false;              // the CPU build runs the two bodies as separate sweeps
-#endif
       if (nbgrad) {
 #ifndef GH_EMU
         tbeg(c, 3);
@@ -3071,7 +3131,7 @@ struct Pipe {
         }
         tend(c, 3);
 #endif
-      } else {
+      } else if (!faces_nb) {
         L2P(c, body_nb, k_nb, (), d.nj, d.nax);
       }
 #ifdef GH_EMU
@@ -3088,7 +3148,8 @@ struct Pipe {
         if (base > d.fcap) d.cnt[CNT_F1OVF]++;
       }
 #else
-      hipLaunchKernelGGL(k_f1_scan, dim3(d.nj), dim3(KB), 0, c->stream, d);
+      bool grad_scan = !d.packed && !nbgrad && !c->f1cell && !d.pc;    // the scan rides with the gradient pass
+      if (!grad_scan) hipLaunchKernelGGL(k_f1_scan, dim3(d.nj), dim3(KB), 0, c->stream, d);
 #endif
       if (c->f1cell) {
         tbeg(c, 5);
@@ -3117,12 +3178,14 @@ struct Pipe {
           bool sph = c->cfg.geom == SPH;
           if (d.packed) {
             if (sph) hipLaunchKernelGGL((k_f1grad<true, NQ, SPH>), persist_grid(c, (const void*)&k_f1grad<true, NQ, SPH>, bs, lds),
-                                        dim3(bs), lds, c->stream, d, d.nax, c->remap);
+                                        dim3(bs), lds, c->stream, d, d.nax, c->remap, 0);
             else hipLaunchKernelGGL((k_f1grad<true, NQ, CART>), persist_grid(c, (const void*)&k_f1grad<true, NQ, CART>, bs, lds),
-                                    dim3(bs), lds, c->stream, d, d.nax, c->remap);
+                                    dim3(bs), lds, c->stream, d, d.nax, c->remap, 0);
           } else {
-            if (sph) hipLaunchKernelGGL((k_f1grad<false, NQ, SPH>), pl.g, dim3(bs), lds, c->stream, d, d.nax, pl.remap);
-            else hipLaunchKernelGGL((k_f1grad<false, NQ, CART>), pl.g, dim3(bs), lds, c->stream, d, d.nax, pl.remap);
+            int y0 = (d.nj + (int)pl.g.x - 1) / (int)pl.g.x;
+            pl.g.y += y0;
+            if (sph) hipLaunchKernelGGL((k_f1grad<false, NQ, SPH>), pl.g, dim3(bs), lds, c->stream, d, d.nax, pl.remap, y0);
+            else hipLaunchKernelGGL((k_f1grad<false, NQ, CART>), pl.g, dim3(bs), lds, c->stream, d, d.nax, pl.remap, y0);
           }
         }
 #endif
@@ -3605,6 +3668,9 @@ int gammahip_load(gammahip_ctx* c, const double* x, const double* dx, const doub
       else hfx[k] = hx[k + 1] - hdx[k + 1] / 2.;
     }
   }
+  c->live = 0;
+  for (int j = 0; j < nj; ++j) c->live += (ntrack[j] + 63) / 64;
+  if (cf.nd == 2 && c->block_auto) c->block = c->live <= BLOCK64_LIVE ? 64 : 128;
   int e = 0;
   e |= h2d(c, d.ntrack, ntrack.data(), sizeof(int) * nj);
   e |= h2d(c, d.trg, trg.data(), sizeof(int) * nj);
@@ -3694,6 +3760,7 @@ int gammahip_set_option(gammahip_ctx* c, int key, long long value) {
     case GAMMAHIP_OPT_BLOCK:
       if (value != 64 && value != 128 && value != 256) return fail(c, "block must be 64, 128 or 256");
       c->block = (int)value;
+      c->block_auto = false;
       build_tiles(c);
       return post(c);
     case GAMMAHIP_OPT_F1FUSE: c->d.f1fused = value ? 1 : 0; return 0;

@@ -171,7 +171,7 @@ int  gammahip_stats_get(gammahip_ctx* ctx, gammahip_stats* st);
 int  gammahip_regrid_counts(gammahip_ctx* ctx, long long* splits, long long* merges);
 /* Average duration (ms) of the dominant kernel launches since the last call,
  * measured with HIP events on the context's stream: entry 0 the update, 1 the
- * MV face pass, 2 the F1 face pass, 3 the transverse-gradient pass, 4 the F1
+ * MV face pass (small 2D grids: with the F1 neighbour search), 2 the F1 face pass, 3 the transverse-gradient pass, 4 the F1
  * flux sums, 5 the fused gradient-and-face pass. */
 int  gammahip_kernel_times(gammahip_ctx* ctx, double* ms_per_launch /* [16] */,
                            long long* launches /* [16] */);
@@ -179,7 +179,7 @@ int  gammahip_sync(gammahip_ctx* ctx);
 
 /* Launch options (no counterpart in the reference; chosen by the autotuner in
  * gamma_amd/autotune.py): threads per workgroup of the per-cell kernels (64,
- * 128, 256; default 128), the order of the (track, chunk) tiles (REMAP 0
+ * 128, 256; default 128, on 2D grids of at most 1024 wavefronts 64), the order of the (track, chunk) tiles (REMAP 0
  * hardware order; 1 XCD-aware bands of tracks; 2 track groups, the default:
  * each workgroup takes one 64-cell chunk of block/64 consecutive tracks, one
  * track per wavefront), replay of
