@@ -2520,10 +2520,13 @@ __global__ void k_mlp_draw(const float4* __restrict__ XT, float4* __restrict__ x
 // Gradient of the mean squared error over the states xb[0..nb), FP32 forward
 // and backward: workgroup b sums tiles b, b + gridDim, ... of TS states into
 // its own row of `part` (NTRAIN entries, then the loss), which k_mlp_adam sums.
-// The three 64-wide products of a tile (hidden layer, its weight gradient, the
-// first layer's error) run as v_mfma_f32_16x16x4_f32 with FP32 accumulation,
-// wavefront v on columns (rows of the weight gradient) 16 v .. 16 v + 15;
-// everything else of a column stays in the lanes that hold it.
+// The hidden layer's weight gradient and the first layer's error run as
+// v_mfma_f32_16x16x4_f32 with FP32 accumulation, wavefront v on columns (rows
+// of the weight gradient) 16 v .. 16 v + 15; everything else of a column stays
+// in the lanes that hold it.  The forward pass keeps forward_f32's order of
+// sums on the vector ALU: a unit within rounding of zero is on or off by it,
+// and each such unit that falls the other way moves a training run by more
+// than all other rounding.
 // The pass is bound by latency (0.1 GFLOP a step): 32 states a tile put 128
 // workgroups on a batch of 4096, and rows stored side by side replace
 // 4481 atomic sums per workgroup at a stride of one line each, which took
@@ -2537,10 +2540,12 @@ __global__ void __launch_bounds__(256) k_mlp_grad(const float* __restrict__ w, c
                                                   int nb, float* __restrict__ part) {
   __shared__ __align__(16) float W2[H * TLD], H1[TS * TLD], Z2[TS * TLD];
   __shared__ float4 xs[TS];
-  __shared__ float yp[4][TS], dys[TS];
+  __shared__ float4 w3s[H / 4];
+  __shared__ float dys[TS];
   int t = (int)threadIdx.x, wv = t >> 6, l = t & 63, c = l & 15, g = l >> 4, col = 16 * wv + c;
   for (int e = t; e < H * H / 4; e += 256)
     *(float4*)&W2[(e >> 4) * TLD + 4 * (e & 15)] = ((const float4*)(w + OW2))[e];
+  if (t < H) ((float*)w3s)[t] = w[OW3 + t];
   float b2 = w[OB2 + col], w3 = w[OW3 + col];
   float b1 = w[OB1 + l], w10 = w[OW1 + 3 * l], w11 = w[OW1 + 3 * l + 1], w12 = w[OW1 + 3 * l + 2];
   floatx4 gw2[4] = {floatx4{}, floatx4{}, floatx4{}, floatx4{}};
@@ -2556,25 +2561,31 @@ __global__ void __launch_bounds__(256) k_mlp_grad(const float* __restrict__ w, c
       H1[(wv * (TS / 4) + q) * TLD + l] = a > 0.f ? a : 0.f;
     }
     __syncthreads();
-    floatx4 z[2] = {floatx4{}, floatx4{}};                   // layer 2: rows 16 m + 4 g + r, column col
-#pragma unroll
-    for (int kk = 0; kk < H / 4; ++kk) {
-      int k = 4 * kk + g;
-      float b = W2[col * TLD + k];
+    float z[2][4];                                           // layer 2: rows 16 m + 4 g + r, column col
+    for (int m = 0; m < 2; ++m)
+      for (int r = 0; r < 4; ++r) z[m][r] = b2;
+#pragma unroll 4
+    for (int k = 0; k < H; k += 4) {
+      float4 u = *(const float4*)&W2[col * TLD + k];
       for (int m = 0; m < 2; ++m)
-        z[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(H1[(16 * m + c) * TLD + k], b, z[m], 0, 0, 0);
+        for (int r = 0; r < 4; ++r) {
+          float4 h = *(const float4*)&H1[(16 * m + 4 * g + r) * TLD + k];
+          z[m][r] += u.x * h.x; z[m][r] += u.y * h.y; z[m][r] += u.z * h.z; z[m][r] += u.w * h.w;
+        }
     }
     for (int m = 0; m < 2; ++m)
       for (int r = 0; r < 4; ++r) {
-        float v = z[m][r] + b2;
-        z[m][r] = v > 0.f ? v : 0.f;
-        float y = w3 * z[m][r];
-        for (int o = 1; o < 16; o <<= 1) y += __shfl_xor(y, o, 64);
-        if (c == 0) yp[wv][16 * m + 4 * g + r] = y;
+        z[m][r] = z[m][r] > 0.f ? z[m][r] : 0.f;
+        Z2[(16 * m + 4 * g + r) * TLD + col] = z[m][r];
       }
     __syncthreads();
     if (t < TS) {
-      float y = w[OB3] + ((yp[0][t] + yp[1][t]) + (yp[2][t] + yp[3][t]));
+      float y = w[OB3];
+#pragma unroll 4
+      for (int k = 0; k < H; k += 4) {
+        float4 h = *(const float4*)&Z2[t * TLD + k], u = w3s[k / 4];
+        y += u.x * h.x; y += u.y * h.y; y += u.z * h.z; y += u.w * h.w;
+      }
       float e = tile * TS + t < nb ? y - xs[t].w : 0.f, dy = 2.f * e / nb;
       dys[t] = dy;
       gb3 += dy;
@@ -2630,7 +2641,7 @@ __global__ void __launch_bounds__(256) k_mlp_grad(const float* __restrict__ w, c
   }
 }
 
-// Sums the workgroups' gradients (four threads an entry), then either stores
+// Sums the workgroups' gradients (four threads an entry, in double), then either stores
 // the sums (gout: the gradient entry point) or takes an Adam step (Kingma & Ba
 // 2015) with bias corrections c1 = 1 - b1^step, c2 = 1 - b2^step; the loss goes
 // to *loss.  In training the workgroups past the parameters gather the next
@@ -2645,17 +2656,17 @@ __global__ void __launch_bounds__(256) k_mlp_adam(const float* __restrict__ part
     mlp_draw(XT, xb, ((int)blockIdx.x - ADAM_WG) * 256 + (int)threadIdx.x, nb, n, seed, step);
     return;
   }
-  __shared__ float sm[4][64];
+  __shared__ double sm[4][64];
   int t = (int)threadIdx.x, k = (int)blockIdx.x * 64 + (t & 63);
-  float gg = 0.f;
+  double sum = 0.;
   if (k <= NTRAIN) {
 #pragma unroll 8
-    for (int b = t >> 6; b < rows; b += 4) gg += part[(long long)b * GROW + k];
+    for (int b = t >> 6; b < rows; b += 4) sum += part[(long long)b * GROW + k];
   }
-  sm[t >> 6][t & 63] = gg;
+  sm[t >> 6][t & 63] = sum;
   __syncthreads();
   if (t >= 64 || k > NTRAIN) return;
-  gg = (sm[0][t] + sm[1][t]) + (sm[2][t] + sm[3][t]);
+  float gg = (float)((sm[0][t] + sm[1][t]) + (sm[2][t] + sm[3][t]));
   if (k == NTRAIN) { *loss = gg; return; }
   if (gout) { gout[k] = gg; return; }
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
@@ -4155,7 +4166,7 @@ int gammahip_mlp_train(const double* states, long long n, float* params, int ste
   unsigned gather = (batch + 255) / 256;
   hipLaunchKernelGGL(k_mlp_draw, dim3(gather), dim3(256), 0, 0, XT, xb, batch, n, seed, 0ll);
   for (int k = 0; k < steps; ++k) {
-    float c1 = (float)(1. - pow((double)0.9f, k + 1)), c2 = (float)(1. - pow((double)0.999f, k + 1));
+    float c1 = 1.f - powf(0.9f, (float)(k + 1)), c2 = 1.f - powf(0.999f, (float)(k + 1));
     hipLaunchKernelGGL(k_mlp_grad, dim3(rows), dim3(256), 0, 0, w, xb, batch, part);
     hipLaunchKernelGGL(k_mlp_adam, dim3(ADAM_WG + (k + 1 < steps ? gather : 0)), dim3(256), 0, 0, part, rows, w, m, v,
                        c1, c2, lr, (float*)nullptr, loss + k, XT, xb, batch, n, seed, (long long)k + 1);
