@@ -141,12 +141,21 @@ def gradient(params: np.ndarray, states: np.ndarray):
     return g, float(loss[0])
 
 
+def _rows(states: np.ndarray) -> np.ndarray:
+    """states as C-contiguous float64 rows of 3 or more: itself where it is that
+    already (the library reads the first three of each row), else the first
+    three columns copied."""
+    if states.dtype == np.float64 and states.flags.c_contiguous and states.ndim == 2 and states.shape[1] >= 3:
+        return states
+    return np.ascontiguousarray(states[:, :3], dtype=np.float64)
+
+
 def infer(params: np.ndarray, states: np.ndarray, mfma: bool = True) -> np.ndarray:
     """Pressure guesses of states [n][>=3]; BF16 MFMA hidden layer or FP32."""
-    st = np.ascontiguousarray(states[:, :3], dtype=np.float64)
+    st = _rows(states)
     w = np.ascontiguousarray(params, dtype=np.float32)
     out = np.zeros(st.shape[0])
-    if _lib().gammahip_mlp_infer(_p(w), _p(st), st.shape[0], _p(out), int(mfma)) != 0:
+    if _lib().gammahip_mlp_infer_ld(_p(w), _p(st), st.shape[1], st.shape[0], _p(out), int(mfma)) != 0:
         raise RuntimeError("gammahip_mlp_infer failed")
     return out
 
@@ -156,7 +165,7 @@ def c2p_batch(states: np.ndarray, guess: np.ndarray, gamma: float, guess2: np.nd
     """FP64 cons2prim of states [n][>=3] from the given starting pressures
     (the kernels' cons2prim; ``lib_path`` may name the CPU build of the same
     bodies)."""
-    st = np.ascontiguousarray(states[:, :3], dtype=np.float64)
+    st = _rows(states)
     n = st.shape[0]
     g = np.ascontiguousarray(guess, dtype=np.float64)
     g2 = None if guess2 is None else np.ascontiguousarray(guess2, dtype=np.float64)
@@ -164,8 +173,8 @@ def c2p_batch(states: np.ndarray, guess: np.ndarray, gamma: float, guess2: np.nd
     it = np.zeros(n, dtype=np.int32)
     fl = np.zeros(n, dtype=np.int32)
     us = np.zeros(n, dtype=np.int32)
-    r = H.load_library(lib_path).gammahip_c2p_batch(_p(st), _p(g), None if g2 is None else _p(g2), n, gamma,
-                                                    solver, maxit, _p(p), _p(it), _p(fl), _p(us))
+    r = H.load_library(lib_path).gammahip_c2p_batch_ld(_p(st), st.shape[1], _p(g), None if g2 is None else _p(g2), n,
+                                                       gamma, solver, maxit, _p(p), _p(it), _p(fl), _p(us))
     if r != 0:
         raise RuntimeError("gammahip_c2p_batch failed")
     return {"p": p, "iters": it, "fail": fl, "used": us}

@@ -241,6 +241,9 @@ int  gammahip_mlp_train(const double* states, long long n, float* params, int st
 int  gammahip_mlp_grad(const float* params, const double* states, int n, float* grad, float* loss);
 int  gammahip_mlp_infer(const float* params, const double* states, long long n, double* p_out,
                         int mfma);
+/* the same on rows of ld >= 3 doubles whose first three are (D, |S|, tau) */
+int  gammahip_mlp_infer_ld(const float* params, const double* states, int ld, long long n, double* p_out,
+                           int mfma);
 /* gammahip_mlp_infer without any allocation (no counterpart in the reference;
  * for callers that cannot allocate device memory: code under HIP graph
  * capture, tight serving loops).  params [gammahip_mlp_nparams()], states
@@ -276,6 +279,15 @@ int  gammahip_mlp_load(gammahip_ctx* ctx, const float* params);
 int  gammahip_c2p_batch(const double* states, const double* guess, const double* guess2, long long n,
                         double gamma, int solver, int maxit, double* p_out, int* iters, int* fail,
                         int* used);
+/* the same on rows of ld >= 3 doubles whose first three are (D, |S|, tau) */
+int  gammahip_c2p_batch_ld(const double* states, int ld, const double* guess, const double* guess2, long long n,
+                           double gamma, int solver, int maxit, double* p_out, int* iters, int* fail,
+                           int* used);
+/* The batch calls on host arrays (gammahip_mlp_infer*, gammahip_c2p_batch*)
+ * keep at most two staging buffers of at most 2 MiB (pinned host memory and
+ * as much device memory) for the next call; this gives them back.  Any thread
+ * may call it at any time: buffers in use stay with their call. */
+int  gammahip_release_workspaces(void);
 
 #ifdef __cplusplus
 }
