@@ -70,6 +70,7 @@ struct Dev {
   int nd, nq, nqs, ngst, nj, nax, jL, jR, fcap, shock, sync, solver, guess, maxit;
   int euler;               // TIMESTEP_ Euler (one update per step) instead of RK3
   int pc;                  // piecewise-constant reconstruction instead of PLM
+  int detect;              // the F1 shock pass also sets the shock flags (detectShock)
   int vpspec;              // VARIABLE_PSPEC_: spectral index from the shock's four-velocity
   int rg_mode;             // bit set of the tracks' regrid rules (1 << RG_*)
   int circ;                // CIRC_REGRID_: splits and merges in pairs with the track's victims
@@ -834,6 +835,7 @@ GH_HD void body_f1_shock(const Dev& d, int j, int i) {
   });
   d.sd[k] = Sd;
   d.pspec[k] = ps;
+  if (d.detect && Sd > d.P.shock_thr) d.shk[k] = 1;
 }
 
 // Net F1 flux of a cell that the update will advance (2d.cpp:974-1036: the
@@ -1263,6 +1265,16 @@ GH_HD void body_inject(const Dev& d, int j, int i) {
   load_v<ND, NQ>(d, d.prim, k, p);
   inject<ND, NQ>(p, d.shk[k] != 0, d.pspec[k], d.P);
   store_v<ND, NQ>(d, d.prim, k, p);
+}
+// what follows the last update of a step, folded into it (stage argument bit
+// 2): the thread's own cell takes its particles, its track's first thread
+// advances the time.  No other thread of the update reads either (the per-cell
+// user hooks do: they keep the separate passes).
+enum { STAGE_TAIL = 4 };
+template <int ND, int NQ>
+GH_HD void body_step_tail(const Dev& d, int j, int i) {
+  if (NQ == 10 && d.sync) body_inject<ND, NQ>(d, j, i);
+  if (i == 0) d.tt[j] += d.tdt[j];
 }
 template <int ND, int NQ>
 GH_HD void body_init_gammas(const Dev& d, int j, int i) {
@@ -1987,9 +1999,12 @@ template <int ND, int NQ, int W, int GEO>
 constexpr int update_waves() { return (W == 1 && ND == 2 && NQ == 6 && GEO == CART) ? 5 : W; }
 template <bool PK, int ND, int NQ, int SV, int W, int GEO>
 __global__ void __launch_bounds__(KB, (update_waves<ND, NQ, W, GEO>())) k_update(Dev d, int ni, int remap, int stage) {
+  int tail = stage & STAGE_TAIL;
+  stage &= 3;
   GH_TILE_LOOP(PK, if (i < ni && j < d.nj) {
     if (stage > 1) body_dt(d, j, i);
     body_update_s<ND, NQ, SV, GEO>(d, j, i, stage);
+    if (tail) body_step_tail<ND, NQ>(d, j, i);
   })
 }
 GH_KERNEL2P((, int ND, int NQ), k_inject, (body_inject<ND, NQ>))
@@ -2379,7 +2394,11 @@ __device__ void wg_regrid(const Dev& d, int j) {
   }
 }
 template <int ND, int NQ>
-__global__ void __launch_bounds__(RGB) k_regrid(Dev d) { wg_regrid<ND, NQ>(d, (int)blockIdx.x); }
+__global__ void __launch_bounds__(RGB) k_regrid(Dev d, int reset) {
+  if (reset)                            // no rule or action reads the shock state
+    for (int i = (int)threadIdx.x; i < d.nax; i += RGB) body_shock_reset(d, (int)blockIdx.x, i);
+  wg_regrid<ND, NQ>(d, (int)blockIdx.x);
+}
 
 // ---- the five passes of a 1D step (see s1_face1) ----
 // begin: one workgroup per track; RG: some track has a regrid rule
@@ -2778,9 +2797,12 @@ struct MlpGuess {
 template <bool PK, int ND, int NQ>
 __global__ void __launch_bounds__(KB) k_update_mlp(Dev d, int ni, int remap, int stage) {
   MlpGuess g{d.mw, (const bf16x8*)d.mw2b, d.mlp_thr, d.P.gamma};
+  int tail = stage & STAGE_TAIL;
+  stage &= 3;
   GH_TILE_LOOP(PK, {
     if (stage > 1 && i < ni && j < d.nj) body_dt(d, j, i);
     body_update_g<ND, NQ, C2P_NEWTON>(d, j, i, stage, i < ni && j < d.nj, g);
+    if (tail && i < ni && j < d.nj) body_step_tail<ND, NQ>(d, j, i);
   })
 }
 
@@ -3287,7 +3309,8 @@ struct Pipe {
     Dev& d = c->d;
     tbeg(c, 0);
 #ifdef GH_EMU
-    L2S(c, (body_update<ND, NQ>), d.nj, d.nax, stage);
+    L2S(c, (body_update<ND, NQ>), d.nj, d.nax, stage & 3);
+    if (stage & STAGE_TAIL) L2(c, (body_step_tail<ND, NQ>), d.nj, d.nax);
 #else
     if (d.mw) L2SP(c, _, k_update_mlp, (, ND, NQ), d.nj, d.nax, stage);
     else {
@@ -3314,7 +3337,8 @@ struct Pipe {
     tend(c, 0);
     std::swap(d.fx, d.fxn);
   }
-  static void regrid(gammahip_ctx* c) {
+  // reset: resetShock in the same launch
+  static void regrid(gammahip_ctx* c, bool reset = false) {
     Dev& d = c->d;
     if (!d.rg_mode) return;
 #ifdef GH_EMU
@@ -3326,8 +3350,9 @@ struct Pipe {
       if (ND == 1)
         for (int i = d.ntrack[j]; i < d.nax; ++i) mirror_slot(d, CI(d, j, i));
     }
+    if (reset) L2(c, body_shock_reset, d.nj, d.nax);
 #else
-    hipLaunchKernelGGL((k_regrid<ND, NQ>), dim3(d.nj), dim3(RGB), 0, c->stream, d);
+    hipLaunchKernelGGL((k_regrid<ND, NQ>), dim3(d.nj), dim3(RGB), 0, c->stream, d, reset ? 1 : 0);
 #endif
   }
   static void apply(gammahip_ctx* c, int what) {
@@ -3342,11 +3367,12 @@ struct Pipe {
     }
   }
   // Grid::evolve (rk3.cpp:12-195)
-  static void evolve(gammahip_ctx* c) {
+  // tail: STAGE_TAIL to fold the end of a step into the last update, or 0
+  static void evolve(gammahip_ctx* c, int tail = 0) {
+    if (c->d.euler) { update(c, 1 | tail); return; }   // Grid::evolve of euler.cpp:12-19
     update(c, 1);
-    if (c->d.euler) return;              // Grid::evolve of euler.cpp:12-19
     ghosts(c); prep(c, false); update(c, 2);
-    ghosts(c); prep(c, false); update(c, 3);
+    ghosts(c); prep(c, false); update(c, 3 | tail);
   }
   // the 1D step in five passes; general otherwise: packed launches, the learned
   // start, Euler steps, event timing of the separate passes, and user hooks
@@ -3424,15 +3450,24 @@ struct Pipe {
         return;
       }
     }
-    regrid(c);
-    apply(c, GAMMAHIP_RESET_SHOCK);
+    // 2D: the regrid's workgroups clear their track's shock state, the F1
+    // shock pass (which visits every live cell last) sets the flags; slots past
+    // a track's end hold -1, above no threshold of -1 or more
+    Dev& d = c->d;
+    bool rs = ND == 2 && d.shock && d.rg_mode, ds = ND == 2 && d.shock && d.P.shock_thr >= -1.;
+    regrid(c, rs);
+    if (!rs) apply(c, GAMMAHIP_RESET_SHOCK);
     ghosts(c, true);          // track lengths settle here: rebuild the tile list
+    d.detect = ds;
     prep(c, false);           // the stage-1 dt candidates: formed by collect_dt
-    apply(c, GAMMAHIP_DETECT_SHOCK);
+    d.detect = 0;
+    if (!ds) apply(c, GAMMAHIP_DETECT_SHOCK);
     collect_dt(c, true);
-    evolve(c);
-    apply(c, GAMMAHIP_ADVANCE_TIME);
-    apply(c, GAMMAHIP_INJECT);
+    evolve(c, d.ucell ? 0 : STAGE_TAIL);
+    if (d.ucell) {
+      apply(c, GAMMAHIP_ADVANCE_TIME);
+      apply(c, GAMMAHIP_INJECT);
+    }
   }
 };
 
