@@ -23,6 +23,7 @@ from __future__ import annotations
 import os
 import shutil
 import subprocess
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -114,11 +115,13 @@ def build_host() -> list:
 
 
 def build_all() -> None:
-    build_hip()
-    build_emu()
-    build_oracle()
+    """Everything; the two builds of the HIP library (about two minutes each)
+    and the CPU pieces side by side."""
+    with ThreadPoolExecutor(4) as ex:
+        jobs = [ex.submit(f) for f in (build_hip, build_hooks_variant, build_emu, build_oracle)]
+        for j in jobs:
+            j.result()
     build_host()
-    build_hooks_variant()
 
 
 if __name__ == "__main__":

@@ -2411,8 +2411,19 @@ __global__ void __launch_bounds__(RG ? RGB : 64) k1_begin(Dev d) {
   }
   if ((int)threadIdx.x < 2 * d.ngst) body_ghost_mv<1, NQ>(d, j, (int)threadIdx.x);
 }
-template <int NQ, bool SHK>
+// STD: constant adiabatic index, piecewise-linear reconstruction, constant
+// spectral index -- the options that run-time switches otherwise keep apart in
+// these kernels, splitting their arithmetic into blocks the compiler cannot
+// merge (a fifth of the instructions: 64-cell track 71.0 -> 68.5 us a step,
+// 4000 cells 128.5 -> 125.4, 256 tracks 774 -> 750; the 2D kernels gain
+// nothing from it, the ten-field face pass loses a wavefront per SIMD).
+GH_HD void s1_options(Dev& d, bool std) {
+  d.ucell = 0;                          // such grids take the general path
+  if (std) { d.P.synge = 0; d.pc = 0; d.vpspec = 0; }
+}
+template <int NQ, bool SHK, bool STD>
 __global__ void __launch_bounds__(S1B) k1_faces(Dev d) {
+  s1_options(d, STD);
   __shared__ double sv[S1B], sl[S1B], sm[S1B / 64];
   int j = (int)blockIdx.y, t = (int)threadIdx.x, i = (int)blockIdx.x * S1C + t - 1;
   int nt = d.ntrack[j];
@@ -2432,8 +2443,9 @@ __global__ void __launch_bounds__(S1B) k1_faces(Dev d) {
     d.tpart[(long long)j * d.s1ch + blockIdx.x] = m;
   }
 }
-template <int NQ, bool SHK, int SV, int STAGE>
+template <int NQ, bool SHK, int SV, int STAGE, bool STD>
 __global__ void __launch_bounds__(S1B) k1_stage(Dev d) {
+  s1_options(d, STD);
   constexpr int NS = NQ - 1;
   __shared__ double sv[S1B], sl[S1B], sx[S1B], sa[S1B], sf[NS][S1B];
   int j = (int)blockIdx.y, t = (int)threadIdx.x, i = (int)blockIdx.x * S1C + t - 1;
@@ -3426,10 +3438,13 @@ struct Pipe {
     dim3 tiles(d.s1ch, d.nj);
     if (d.rg_mode) hipLaunchKernelGGL((k1_begin<NQ, true>), dim3(d.nj), dim3(RGB), 0, c->stream, d);
     else hipLaunchKernelGGL((k1_begin<NQ, false>), dim3(d.nj), dim3(64), 0, c->stream, d);
-    hipLaunchKernelGGL((k1_faces<NQ, SHK>), tiles, dim3(S1B), 0, c->stream, d);
+    bool std = !d.P.synge && !d.pc && !d.vpspec;
+    if (std) hipLaunchKernelGGL((k1_faces<NQ, SHK, true>), tiles, dim3(S1B), 0, c->stream, d);
+    else hipLaunchKernelGGL((k1_faces<NQ, SHK, false>), tiles, dim3(S1B), 0, c->stream, d);
     auto stage = [&](auto st, auto sv) {
       constexpr int ST = decltype(st)::value, SV = decltype(sv)::value;
-      hipLaunchKernelGGL((k1_stage<NQ, SHK, SV, ST>), tiles, dim3(S1B), 0, c->stream, d);
+      if (std) hipLaunchKernelGGL((k1_stage<NQ, SHK, SV, ST, true>), tiles, dim3(S1B), 0, c->stream, d);
+      else hipLaunchKernelGGL((k1_stage<NQ, SHK, SV, ST, false>), tiles, dim3(S1B), 0, c->stream, d);
       swap();
     };
 #endif
