@@ -2864,6 +2864,13 @@ struct KTimer {
 // 457 -> 418; 512 x 129 (1197) 265 -> 277, its two adjacent tracks in one
 // workgroup reading the same lines.
 constexpr long long FACES_NB_LIVE = 3072, BLOCK64_LIVE = 1024;
+// F1 flux sums inside the update (no pass of their own): with ten fields always
+// (1024 tracks 4187 -> 4119 us a step, 48 tracks 411 -> 398: the update holds
+// 2 to 3 wavefronts per SIMD either way), with six from 512 to 8192 wavefronts
+// (256 x 160 cells 230 -> 228, 512 x 129 262 -> 258, 512 x 256 341 -> 335,
+// 1024 x 512 716 either way; 96 x 33 199 -> 201, 2048 x 2048 4224 -> 4372, where
+// the sums' gathers wait longer in the update than in a light pass).
+bool f1_sums_in_update(int nq, long long live) { return nq == 10 || (live >= 512 && live <= 8192); }
 
 struct gammahip_ctx {
   gammahip_config cfg;
@@ -2883,6 +2890,7 @@ struct gammahip_ctx {
   int block = 128;         // threads per workgroup of the per-cell kernels (64..256)
   bool block_auto = true;  // block follows BLOCK64_LIVE until the option sets it (2D)
   long long live = 0;      // wavefronts of 64 live cells at load
+  bool f1fuse_auto = true; // F1 sums in the update by f1_sums_in_update until the option says so
   int remap = 2;           // tile order: 0 hardware, 1 XCD bands, 2 track groups
   int use_graph = 0;       // replay steps from a captured hipGraph
   int persist = 0;         // packed launch: at most this many persistent workgroups per CU (0: off),
@@ -3866,6 +3874,7 @@ int gammahip_load(gammahip_ctx* c, const double* x, const double* dx, const doub
   }
   c->live = 0;
   for (int j = 0; j < nj; ++j) c->live += (ntrack[j] + 63) / 64;
+  if (cf.nd == 2 && c->f1fuse_auto) d.f1fused = f1_sums_in_update(cf.nq, c->live) ? 1 : 0;
   if (cf.nd == 2 && c->block_auto) c->block = c->live <= BLOCK64_LIVE ? 64 : 128;
   int e = 0;
   e |= h2d(c, d.ntrack, ntrack.data(), sizeof(int) * nj);
@@ -3959,7 +3968,7 @@ int gammahip_set_option(gammahip_ctx* c, int key, long long value) {
       c->block_auto = false;
       build_tiles(c);
       return post(c);
-    case GAMMAHIP_OPT_F1FUSE: c->d.f1fused = value ? 1 : 0; return 0;
+    case GAMMAHIP_OPT_F1FUSE: c->d.f1fused = value ? 1 : 0; c->f1fuse_auto = false; return 0;
     case GAMMAHIP_OPT_F1CELL: c->f1cell = value ? 1 : 0; return 0;
     case GAMMAHIP_OPT_FUSE:
       if (value < 0 || value > 7) return fail(c, "fuse option must be in 0..7");

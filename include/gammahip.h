@@ -194,7 +194,8 @@ int  gammahip_sync(gammahip_ctx* ctx);
  * runs the F1 face kernel in a build capped at 128 registers (4 wavefronts
  * per SIMD) with six fields, at 168 (3) with ten, bit 1 the update kernel in
  * one capped at 96 (5 wavefronts; the default build of 2D Cartesian six-field
- * grids), spilling what does not fit; F1FUSE 1 sums each cell's F1 face fluxes inside
+ * grids), spilling what does not fit; F1FUSE 1 (the
+ * default with ten fields, and with six on grids of 512 to 8192 wavefronts) sums each cell's F1 face fluxes inside
  * the update kernel instead of in a pass of its own (fewer bytes, a longer
  * dependent-load chain in the update); SOLVER switches cons2prim between
  * Brent (0, the reference's algorithm) and Newton (1; required while the
