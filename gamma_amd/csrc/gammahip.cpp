@@ -3205,7 +3205,8 @@ struct Pipe {
         if (base > d.fcap) d.cnt[CNT_F1OVF]++;
       }
 #else
-      bool grad_scan = !d.packed && !nbgrad && !c->f1cell && !d.pc;    // the scan rides with the gradient pass
+      // the scan rides with the gradient pass, where its rows fit the grid
+      bool grad_scan = !d.packed && !nbgrad && !c->f1cell && !d.pc && d.nj <= 32767;
       if (!grad_scan) hipLaunchKernelGGL(k_f1_scan, dim3(d.nj), dim3(KB), 0, c->stream, d);
 #endif
       if (c->f1cell) {
@@ -3239,7 +3240,7 @@ struct Pipe {
             else hipLaunchKernelGGL((k_f1grad<true, NQ, CART>), persist_grid(c, (const void*)&k_f1grad<true, NQ, CART>, bs, lds),
                                     dim3(bs), lds, c->stream, d, d.nax, c->remap, 0);
           } else {
-            int y0 = (d.nj + (int)pl.g.x - 1) / (int)pl.g.x;
+            int y0 = grad_scan ? (d.nj + (int)pl.g.x - 1) / (int)pl.g.x : 0;
             pl.g.y += y0;
             if (sph) hipLaunchKernelGGL((k_f1grad<false, NQ, SPH>), pl.g, dim3(bs), lds, c->stream, d, d.nax, pl.remap, y0);
             else hipLaunchKernelGGL((k_f1grad<false, NQ, CART>), pl.g, dim3(bs), lds, c->stream, d, d.nax, pl.remap, y0);
@@ -3402,7 +3403,8 @@ struct Pipe {
   // that read the track's time while a stage runs
   static bool fused1(const gammahip_ctx* c) {
     const Dev& d = c->d;
-    return ND == 1 && !d.packed && !d.mw && !d.euler && !d.ucell && !c->timing && !c->user_hooks;
+    return ND == 1 && !d.packed && !d.mw && !d.euler && !d.ucell && !c->timing && !c->user_hooks &&
+           d.nj <= 65535;               // tracks are the grid's second dimension
   }
   template <bool SHK>
   static void step1(gammahip_ctx* c) {
@@ -3807,6 +3809,7 @@ int gammahip_load(gammahip_ctx* c, const double* x, const double* dx, const doub
   const gammahip_config& cf = c->cfg;
   int nj = d.nj, nax = d.nax, ng = d.ngst, nm = cf.ncell_mv, na = cf.ntracks_active;
   size_t cs = d.cs;
+  drop_graph(c);            // the rules below pick launches by the tracks' hooks and lengths
   c->user_hooks = false;
   // host images of the initial state (Cinit + mpi_distribute, 1d.cpp:956-969, 2d.cpp:1175-1195)
   std::vector<int> ntrack(nj, nm + 2 * ng), tgeom(nj), tkin(nj), tbnd(nj), trg(nj, RG_NONE);
