@@ -1081,7 +1081,7 @@ GH_HD void body_update(const Dev& d, int j, int i, int stage) {
 // to memory in the last stage only: nothing reads the others' outside the pass.
 
 // The stage passes write live cells only: slots past a track's end hold the
-// same values in both sets of planes (load, restore and regrid see to it), as
+// same values in both sets of planes (load, restore, INIT_GAMMAS and regrid see to it), as
 // they would if the cells were advanced in place.
 GH_HD void mirror_slot(const Dev& d, long long k) {
   for (int s = 0; s < d.nqs; ++s) d.primn[s * d.cs + k] = d.prim[s * d.cs + k];
@@ -3908,7 +3908,6 @@ int gammahip_load(gammahip_ctx* c, const double* x, const double* dx, const doub
   e |= h2d(c, d.cdx, hdx.data(), sizeof(double) * cs);
   e |= h2d(c, d.fx, hfx.data(), sizeof(double) * cs);
   e |= h2d(c, d.dtloc, hdt.data(), sizeof(double) * cs);
-  if (e || mirror_state(c)) return -1;
   if (d.shock) {
     std::vector<double> m1(cs, -1.);
     e |= h2d(c, d.sd, m1.data(), sizeof(double) * cs);
@@ -3920,6 +3919,7 @@ int gammahip_load(gammahip_ctx* c, const double* x, const double* dx, const doub
     P.ghosts(c, true);
   });
   if (r) return r;
+  if (mirror_state(c)) return -1;   // after INIT_GAMMAS, which writes unused slots too
   return post(c);
 }
 
@@ -4044,7 +4044,10 @@ int gammahip_regrid(gammahip_ctx* c) { drop_graph(c); return dispatch(c, [&](aut
 int gammahip_update_ghosts(gammahip_ctx* c) { drop_graph(c); return dispatch(c, [&](auto P) { P.ghosts(c, true); }) || post(c); }
 int gammahip_prep_for_update(gammahip_ctx* c) { drop_graph(c); return dispatch(c, [&](auto P) { P.prep(c); }) || post(c); }
 int gammahip_evolve(gammahip_ctx* c) { drop_graph(c); return dispatch(c, [&](auto P) { P.evolve(c); }) || post(c); }
-int gammahip_apply(gammahip_ctx* c, int what) { drop_graph(c); return dispatch(c, [&](auto P) { P.apply(c, what); }) || post(c); }
+int gammahip_apply(gammahip_ctx* c, int what) {
+  drop_graph(c);
+  return dispatch(c, [&](auto P) { P.apply(c, what); }) || (what == GAMMAHIP_INIT_GAMMAS && mirror_state(c)) || post(c);
+}
 
 int gammahip_collect_dt(gammahip_ctx* c, double* dt_out) {
   drop_graph(c);
