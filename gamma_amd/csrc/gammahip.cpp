@@ -2719,8 +2719,13 @@ __global__ void __launch_bounds__(256) k_mlp_adam(const float* __restrict__ part
 // path is bound by the vector ALU (about 1200 instructions per 64 states: 64
 // first-layer units in the rounding order of the FP32 sum, the output layer,
 // three logarithms and an exponential in FP64): 2^20 states 77 -> 35 us.
+// The FP32 path packs nothing for a workgroup to share, so it takes one
+// wavefront a workgroup, which spreads small batches over the most CUs (64
+// against 256 threads: 1 to 3000 states 26.0-26.8 against 29.2-30.6 us, 10,000
+// 26.9 against 30.9, from 65,536 on alike).
+constexpr int infer_threads(bool mfma) { return mfma ? 256 : 64; }
 template <bool MFMA>
-__global__ void __launch_bounds__(256, MFMA ? 4 : 1) k_mlp_infer(const float* __restrict__ w,
+__global__ void __launch_bounds__(infer_threads(MFMA), MFMA ? 4 : 1) k_mlp_infer(const float* __restrict__ w,
                                                                  const double* __restrict__ st, long long n,
                                                                  double* __restrict__ out) {
   __shared__ float4 u1[MFMA ? H : 1], u2[MFMA ? H / 4 : 1], u3[MFMA ? H / 4 : 1];
@@ -2741,7 +2746,8 @@ __global__ void __launch_bounds__(256, MFMA ? 4 : 1) k_mlp_infer(const float* __
     }
     __syncthreads();
   }
-  for (long long s0 = (long long)blockIdx.x * 256; s0 < n; s0 += MFMA ? (long long)gridDim.x * 256 : n) {
+  constexpr int WG = infer_threads(MFMA);
+  for (long long s0 = (long long)blockIdx.x * WG; s0 < n; s0 += MFMA ? (long long)gridDim.x * WG : n) {
     long long s = s0 + t;
     bool valid = s < n;
     double D = valid ? st[3 * s] : 1., S = valid ? st[3 * s + 1] : 0., tau = valid ? st[3 * s + 2] : 1.;
@@ -2760,12 +2766,13 @@ __global__ void __launch_bounds__(256, MFMA ? 4 : 1) k_mlp_infer(const float* __
 }
 // at most 2048 workgroups, each packing once: two rounds of the 4 a CU that the
 // registers admit, which balance better than one (4 M states 133 against 140 us);
-// the FP32 path has nothing to save and takes a workgroup per 256 states
+// the FP32 path has nothing to save and takes a workgroup per 64 states
 constexpr long long INFER_WG = 2048;
 void launch_infer(const float* w, const double* st, long long n, double* out, int mfma, hipStream_t s) {
-  long long g = (n + 255) / 256;
-  if (mfma) hipLaunchKernelGGL(k_mlp_infer<true>, dim3((unsigned)std::min(g, INFER_WG)), dim3(256), 0, s, w, st, n, out);
-  else hipLaunchKernelGGL(k_mlp_infer<false>, dim3((unsigned)g), dim3(256), 0, s, w, st, n, out);
+  int t = infer_threads(mfma != 0);
+  long long g = (n + t - 1) / t;
+  if (mfma) hipLaunchKernelGGL(k_mlp_infer<true>, dim3((unsigned)std::min(g, INFER_WG)), dim3(t), 0, s, w, st, n, out);
+  else hipLaunchKernelGGL(k_mlp_infer<false>, dim3((unsigned)g), dim3(t), 0, s, w, st, n, out);
 }
 
 __global__ void k_c2p_batch(const double* __restrict__ st, const double* __restrict__ guess,
