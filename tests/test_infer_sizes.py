@@ -1,6 +1,9 @@
 """Batch inference of device arrays in one launch, at counts either side of a
-wavefront and a workgroup (FP32 path): a state's answer has the bits it
-has in a short batch."""
+wavefront and a workgroup (FP32 path) and past one and two rounds of the
+matrix-instruction path's 2048 workgroups of 256 states, whose walk over its
+share reuses the network packed on chip: a state's answer has the bits it has
+in a short batch.  The library keeps no device memory between calls (the
+network is packed by each workgroup for itself)."""
 from __future__ import annotations
 
 import numpy as np
@@ -10,10 +13,12 @@ from gamma_amd import hip, surrogate as SG
 from test_zz_no_alloc import _Dev, _hip, _params
 
 G53 = 5.0 / 3.0
+ROUND = 2048 * 256
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("mfma,n", [(0, 1), (0, 63), (0, 64), (0, 65), (0, 257), (0, 20_001)])
+@pytest.mark.parametrize("mfma,n", [(0, 1), (0, 63), (0, 64), (0, 65), (0, 257), (0, 20_001),
+                                    (1, ROUND), (1, ROUND + 3), (1, 2 * ROUND + 300)])
 def test_gpu_inference_counts_in_one_launch(mfma, n):
     L, R = hip.load_library(), _hip()
     w = _params(5)
