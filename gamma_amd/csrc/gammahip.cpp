@@ -55,6 +55,8 @@ enum { KIN_NONE = 0, KIN_FIXED = 1, KIN_USER = 2 };
 enum { BND_NONE = 0, BND_BM = 1, BND_USER = 2 };
 enum { RG_NONE = 0, RG_AR2D = 1, RG_BM1D = 2, RG_USER = 3 };
 
+constexpr int RGB = 512;      // threads of the regrid's workgroups
+constexpr int RGS = 4 * RGB;  // its screen, where that runs on its own: a workgroup takes a multiple of this many slots
 constexpr int DT_CH = 1024;   // cells per workgroup of the per-track dt minimum
 // A tile is S1B - 1 cells: thread t takes face and cell tile*(S1B-1) + t - 1,
 // thread 0 only the left face of the tile's first cell, which the tile before
@@ -84,6 +86,8 @@ struct Dev {
   unsigned char* rgflag;   // [nj][nax] the regrid screen's decision per active cell (1: an admissible action)
   double *tvin, *tvout, *tbm, *ty, *tdy, *tdt, *tt, *tmin;
   double *tpart;           // [nj][dtch] dt minimum of each chunk of DT_CH cells of each track
+  int* rgpart;             // [nj][rgch][3] what k_rg_screen found: last cell past the shock threshold, first and last flagged
+  int rgch, rgspan;        // k_rg_screen: workgroups per track (0: k_regrid screens its track itself), slots of each
   int dtch;                // chunks per track: ceil(nax / DT_CH)
   int s1ch;                // 1D: tiles per track of the stage passes, ceil(nax / S1C); tpart is [nj][s1ch] there
   // cells
@@ -1531,15 +1535,18 @@ GH_HD void body_rg_shockpos(const Dev& d, int j, int i) {
   if (i < iL + 1 || i > iR - 1) return;
   if (d.prim[PPP * d.cs + CI(d, j, i)] > 1.5 * d.rg[3] && i > d.tiS[j]) d.tiS[j] = i;
 }
+// whether decision a about cell i of the track at b is admissible at length nt, kept in rgflag
+GH_HD bool rg_flag(const Dev& d, long long b, int i, int nt, int a) {
+  bool ok = (a == RG_SPLIT && nt < d.nax - 1) || (a == RG_MERGE && nt > 2 * d.ngst + 2);
+  d.rgflag[b + i] = ok ? 1 : 0;
+  return ok;
+}
 template <int ND, int NQ>
 GH_HD void body_rg_screen(const Dev& d, int j, int i) {
   if (!active_track(d, j) || d.trg[j] == RG_NONE) return;
   int nt = d.ntrack[j], iL = d.ngst - 1, iR = nt - d.ngst;
   if (i < iL + 1 || i > iR - 1) return;
-  int a = rg_check<ND, NQ>(d, j, i, (double)d.tiS[j]);
-  bool ok = (a == RG_SPLIT && nt < d.nax - 1) || (a == RG_MERGE && nt > 2 * d.ngst + 2);
-  d.rgflag[CI(d, j, i)] = ok ? 1 : 0;
-  if (ok) {
+  if (rg_flag(d, CI(d, j, 0), i, nt, rg_check<ND, NQ>(d, j, i, (double)d.tiS[j]))) {
     GH_ATOMIC_MIN(&d.tfirst[j], i);
     GH_ATOMIC_MAX(&d.tlast[j], i);
   }
@@ -2105,7 +2112,6 @@ __global__ void __launch_bounds__(KB) k_dt_finish(Dev d) {
 // in chunks of RGB cells, each chunk read into registers before any of it is
 // written, chunks taken from the far end towards the action, which is the
 // order in which the sequential loops copy.
-constexpr int RGB = 512;
 template <int ND, int NQ>
 struct CellRec {
   static constexpr int NS = ND == 1 ? NQ - 1 : NQ;
@@ -2246,67 +2252,85 @@ __device__ void wg_merge(const Dev& d, int j, long long b, int i, int* s_left) {
   }
   __syncthreads();
 }
-// One pass over the workgroup's track ahead of the loop: every active cell's
-// decision (rgflag), the shock index and the first and last flagged cell, all
-// of body_rg_shockpos and body_rg_screen.  A decision depends on the shock
-// index only in the nine cells past it, so the cells are read once, judged
-// without that window, and the window judged again when the index is known.
+// The decisions of active cells lo .. hi of track j (rgflag), the last one past
+// the shock threshold and the first and last flagged, taken into best, f and l
+// by the workgroup's threads.  A decision depends on the shock index only in
+// the nine cells past it, so the cells are read once and judged without that
+// window (wg_screen).
+template <int ND, int NQ>
+__device__ void wg_judge(const Dev& d, int j, bool bm, int lo, int hi, int& best, int& f, int& l) {
+  int nt = d.ntrack[j], iR = nt - d.ngst, t = (int)threadIdx.x;
+  long long b = CI(d, j, 0);
+  double thr = 1.5 * d.rg[3];
+  auto flag = [&](int i, int a) {
+    if (!rg_flag(d, b, i, nt, a)) return;
+    f = f < i ? f : i;
+    l = i > l ? i : l;
+  };
+  if (d.trg[j] == RG_USER) {
+    for (int i = lo + t; i <= hi; i += RGB) flag(i, rg_check<ND, NQ>(d, j, i, HUGE_VAL));
+    return;
+  }
+  // U cells of a thread at a time, all read before the first is judged
+  constexpr int U = 4;
+  double rOut = d.cx[b + iR - 1], dy = d.tdy[j];
+  for (int i = lo + t; i <= hi; i += U * RGB) {
+    double dx[U], pp[U], p[U][NQ];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      long long k = b + (i + u * RGB <= hi ? i + u * RGB : i);
+      dx[u] = d.cdx[k];
+      if (bm) {
+        pp[u] = d.prim[PPP * d.cs + k];
+        p[u][UU1] = d.prim[UU1 * d.cs + k];
+        if (ND == 2) p[u][UU2] = d.prim[UU2 * d.cs + k];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      int m = i + u * RGB;
+      if (m > hi) break;
+      if (bm && pp[u] > thr && m > best) best = m;
+      flag(m, bm ? rg_rule_bm(d, dx[u], lfac<ND, NQ>(p[u]), -HUGE_VAL, rOut) : rg_rule_ar(d, dx[u], dy));
+    }
+  }
+}
+// One pass over the workgroup's track ahead of the loop: body_rg_shockpos and
+// body_rg_screen.  The shock index is exact; i0 .. i1 hold every flagged cell,
+// but cells that only the window unflagged may lie at their ends (the loop
+// goes by rgflag, or judges the cells itself).
 // One launch instead of four (clear, shock position, screen, loop): a regrid
 // without actions takes 8 instead of 17 us on one 4000-cell track, 39 instead
 // of 62 us on 256 tracks of 512-16384 cells, 30 us either way on 2048 x 2048.
 template <int ND, int NQ>
 __device__ bool wg_screen(const Dev& d, int j, bool bm, int* red, int* i0, int* i1, double* iS) {
   int nt = d.ntrack[j], iL = d.ngst - 1, iR = nt - d.ngst, t = (int)threadIdx.x;
-  long long b = CI(d, j, 0);
-  double thr = 1.5 * d.rg[3];
-  auto flag = [&](int i, int a) {
-    bool ok = (a == RG_SPLIT && nt < d.nax - 1) || (a == RG_MERGE && nt > 2 * d.ngst + 2);
-    d.rgflag[b + i] = ok ? 1 : 0;
-    return ok ? 1 : 0;
-  };
-  int any = 0, best = iL + 1, mode = d.trg[j];
-  if (mode == RG_USER) {
-    for (int i = iL + 1 + t; i <= iR - 1; i += RGB) any |= flag(i, rg_check<ND, NQ>(d, j, i, HUGE_VAL));
-  } else {
-    // U cells of a thread at a time, all read before the first is judged
-    constexpr int U = 4;
-    double rOut = d.cx[b + iR - 1], dy = d.tdy[j];
-    for (int i = iL + 1 + t; i <= iR - 1; i += U * RGB) {
-      double dx[U], pp[U], p[U][NQ];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        long long k = b + (i + u * RGB <= iR - 1 ? i + u * RGB : i);
-        dx[u] = d.cdx[k];
-        if (bm) {
-          pp[u] = d.prim[PPP * d.cs + k];
-          p[u][UU1] = d.prim[UU1 * d.cs + k];
-          if (ND == 2) p[u][UU2] = d.prim[UU2 * d.cs + k];
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        int m = i + u * RGB;
-        if (m > iR - 1) break;
-        if (bm && pp[u] > thr) best = m;
-        any |= flag(m, bm ? rg_rule_bm(d, dx[u], lfac<ND, NQ>(p[u]), -HUGE_VAL, rOut) : rg_rule_ar(d, dx[u], dy));
-      }
+  int best = iL + 1, f = INT_MAX, l = -1;
+  if (d.rgch) {                         // k_rg_screen has judged the cells
+    for (int q = t; q < d.rgch; q += RGB) {
+      const int* p = d.rgpart + 3 * ((long long)j * d.rgch + q);
+      best = p[0] > best ? p[0] : best;
+      f = p[1] < f ? p[1] : f;
+      l = p[2] > l ? p[2] : l;
     }
+  } else {
+    wg_judge<ND, NQ>(d, j, bm, iL + 1, iR - 1, best, f, l);
   }
   *iS = 0.;
   if (bm) {
     int s = wg_reduce<true>(best, red);
     *iS = (double)s;
     int m = s + 1 + t;
-    if (t < 9 && m <= iR - 1) any |= flag(m, rg_check<ND, NQ>(d, j, m, *iS));
+    if (t < 9 && m <= iR - 1 && rg_flag(d, CI(d, j, 0), m, nt, rg_check<ND, NQ>(d, j, m, *iS))) {
+      f = m < f ? m : f;
+      l = m > l ? m : l;
+    }
   }
-  if (!wg_reduce<true>(any, red)) return false;
-  int f = INT_MAX, l = -1;
-  for (int i = iL + 1 + t; i <= iR - 1; i += RGB)
-    if (d.rgflag[b + i]) { f = f < i ? f : i; l = i; }
   *i0 = wg_reduce<false>(f, red);
+  if (*i0 == INT_MAX) return false;
   *i1 = wg_reduce<true>(l, red);
   __syncthreads();
-  return *i1 >= 0;
+  return true;
 }
 template <int ND, int NQ>
 __device__ void wg_regrid(const Dev& d, int j) {
@@ -2396,9 +2420,32 @@ __device__ void wg_regrid(const Dev& d, int j) {
     for (int m = d.ntrack[j] + (int)threadIdx.x; m < ntmax; m += RGB) mirror_slot(d, b + m);
   }
 }
+// wg_screen's pass over the cells on grids of few long tracks
+// (rg_screen_chipwide): a workgroup for every rgspan slots of a track
+template <int ND, int NQ>
+__global__ void __launch_bounds__(RGB) k_rg_screen(Dev d, int reset) {
+  __shared__ int red[RGB / 64][3];
+  int j = (int)blockIdx.x / d.rgch, s0 = ((int)blockIdx.x - j * d.rgch) * d.rgspan, t = (int)threadIdx.x;
+  if (reset)
+    for (int i = s0 + t; i < s0 + d.rgspan; i += RGB) body_shock_reset(d, j, i);
+  if (!active_track(d, j) || d.trg[j] == RG_NONE) return;
+  int iL = d.ngst - 1, iR = d.ntrack[j] - d.ngst, v[3] = {iL + 1, -INT_MAX, -1};   // best, -first, last
+  int lo = max(s0, iL + 1), hi = min(s0 + d.rgspan, iR) - 1, f = INT_MAX;
+  if (lo <= hi) wg_judge<ND, NQ>(d, j, d.trg[j] == RG_BM1D, lo, hi, v[0], f, v[2]);
+  v[1] = -f;
+  for (int o = 32; o > 0; o >>= 1)
+    for (int q = 0; q < 3; ++q) v[q] = max(v[q], __shfl_xor(v[q], o, 64));
+  if ((t & 63) == 0)
+    for (int q = 0; q < 3; ++q) red[t >> 6][q] = v[q];
+  __syncthreads();
+  if (t >= 3) return;
+  int m = red[0][t];
+  for (int w = 1; w < RGB / 64; ++w) m = max(m, red[w][t]);
+  d.rgpart[3 * (long long)blockIdx.x + t] = t == 1 ? -m : m;
+}
 template <int ND, int NQ>
 __global__ void __launch_bounds__(RGB) k_regrid(Dev d, int reset) {
-  if (reset)                            // no rule or action reads the shock state
+  if (reset && !d.rgch)                 // no rule or action reads the shock state
     for (int i = (int)threadIdx.x; i < d.nax; i += RGB) body_shock_reset(d, (int)blockIdx.x, i);
   wg_regrid<ND, NQ>(d, (int)blockIdx.x);
 }
@@ -2881,6 +2928,23 @@ constexpr long long FACES_NB_LIVE = 3072, BLOCK64_LIVE = 1024;
 // 1024 x 512 716 either way; 96 x 33 199 -> 201, 2048 x 2048 4224 -> 4372, where
 // the sums' gathers wait longer in the update than in a light pass).
 bool f1_sums_in_update(int nq, long long live) { return nq == 10 || (live >= 512 && live <= 8192); }
+
+// The regrid's screen in a launch of its own over the whole chip, on grids of
+// few long tracks (longest: cells of the longest at load), where one workgroup
+// would walk its track while most of the chip idles.  The rules that read the
+// cell's state pay from some 5000 cells, the aspect ratio (the width alone)
+// from 9000, both later the more tracks already fill the chip.  A regrid
+// without actions, one workgroup a track against chip-wide, us:
+// Blandford-McKee rule, 1 track of 4000 cells 8.8 / 9.7, 8000 13.4 / 9.7, 32000
+// 39 / 9.8, a million 1104 / 12.7; 64 tracks of 8000 14.6 / 12.7; 128 of 8000
+// 15.5 / 15.7, 16000 26.6 / 22.3; 256 of 16000 28.9 / 36.4.  Aspect ratio, 9
+// tracks of 8000 8.0 / 8.0, 16000 12.3 / 8.1; 64 of 8000 8.4 / 8.9, 16000
+// 12.6 / 10.8; 128 of 16000 12.9 / 13.0, 32000 24.8 / 18.3; 160 of 16000
+// 13.0 / 14.3.
+bool rg_screen_chipwide(int rg_modes, int tracks, int longest) {
+  double from = (rg_modes & ~(1 << RG_AR2D)) ? 5000. : 9000.;
+  return rg_modes && tracks <= 160 && longest > from * (1. + tracks / 128.);
+}
 
 struct gammahip_ctx {
   gammahip_config cfg;
@@ -3368,6 +3432,12 @@ struct Pipe {
     tend(c, 0);
     std::swap(d.fx, d.fxn);
   }
+#ifndef GH_EMU
+  static void rg_screen(gammahip_ctx* c, bool reset) {
+    Dev& d = c->d;
+    if (d.rgch) hipLaunchKernelGGL((k_rg_screen<ND, NQ>), dim3(d.nj * d.rgch), dim3(RGB), 0, c->stream, d, reset ? 1 : 0);
+  }
+#endif
   // reset: resetShock in the same launch
   static void regrid(gammahip_ctx* c, bool reset = false) {
     Dev& d = c->d;
@@ -3383,6 +3453,7 @@ struct Pipe {
     }
     if (reset) L2(c, body_shock_reset, d.nj, d.nax);
 #else
+    rg_screen(c, reset);
     hipLaunchKernelGGL((k_regrid<ND, NQ>), dim3(d.nj), dim3(RGB), 0, c->stream, d, reset ? 1 : 0);
 #endif
   }
@@ -3456,6 +3527,7 @@ struct Pipe {
     };
 #else
     dim3 tiles(d.s1ch, d.nj);
+    if (d.rg_mode) rg_screen(c, false);
     if (d.rg_mode) hipLaunchKernelGGL((k1_begin<NQ, true>), dim3(d.nj), dim3(RGB), 0, c->stream, d);
     else hipLaunchKernelGGL((k1_begin<NQ, false>), dim3(d.nj), dim3(64), 0, c->stream, d);
     bool std = !d.P.synge && !d.pc && !d.vpspec;
@@ -3759,6 +3831,7 @@ int gammahip_create(const gammahip_config* cfg, gammahip_ctx** out) {
   e |= dalloc(c, &d.tbnd, nj); e |= dalloc(c, &d.tfirst, nj); e |= dalloc(c, &d.tiS, nj);
   e |= dalloc(c, &d.tlast, nj);
   e |= dalloc(c, &d.rgflag, (size_t)cs);
+  e |= dalloc(c, &d.rgpart, 3 * nj * (size_t)((d.nax + RGS - 1) / RGS));
   e |= dalloc(c, &d.tvin, nj); e |= dalloc(c, &d.tvout, nj); e |= dalloc(c, &d.tbm, 4 * nj);
   e |= dalloc(c, &d.ty, nj); e |= dalloc(c, &d.tdy, nj); e |= dalloc(c, &d.tdt, nj);
   e |= dalloc(c, &d.tt, nj); e |= dalloc(c, &d.tmin, nj);
@@ -3887,6 +3960,12 @@ int gammahip_load(gammahip_ctx* c, const double* x, const double* dx, const doub
   }
   c->live = 0;
   for (int j = 0; j < nj; ++j) c->live += (ntrack[j] + 63) / 64;
+  d.rgch = 0;
+  if (rg_screen_chipwide(d.rg_mode, nj, *std::max_element(ntrack.begin(), ntrack.end()))) {
+    long long units = (d.nax + RGS - 1) / RGS;           // about 1024 workgroups: four a CU
+    d.rgspan = RGS * (int)(1 + nj * units / 1024);
+    d.rgch = (d.nax + d.rgspan - 1) / d.rgspan;
+  }
   if (cf.nd == 2 && c->f1fuse_auto) d.f1fused = f1_sums_in_update(cf.nq, c->live) ? 1 : 0;
   if (cf.nd == 2 && c->block_auto) c->block = c->live <= BLOCK64_LIVE ? 64 : 128;
   int e = 0;
