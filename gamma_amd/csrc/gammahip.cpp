@@ -1874,11 +1874,10 @@ __global__ void __launch_bounds__(KB, (SHK || NQ > 6) ? 1 : 5) k_faces_nb(Dev d,
   if (b & 8) body_nb_lanes(d, j, i, in);
   else if (in) body_faces_s<2, NQ, SHK>(d, j, i);
 }
-// exclusive prefix sum of upper-neighbour counts along each track (F1 face slots)
-// inclusive prefix sum of one value per thread over the workgroup: shuffles
-// within each wavefront, the wavefront totals through LDS; *total = the sum
-// over the workgroup
-__device__ int wg_scan_incl(int v, int* wsum, int* total) {
+// inclusive prefix sum of one value per thread over the workgroup of B threads:
+// shuffles within each wavefront, the wavefront totals through LDS; *total =
+// the sum over the workgroup
+__device__ __forceinline__ int wg_scan_incl(int v, int* wsum, int* total, int B) {
   int lane = (int)(threadIdx.x & 63), w = (int)(threadIdx.x >> 6);
   for (int o = 1; o < 64; o <<= 1) {
     int t = __shfl_up(v, o, 64);
@@ -1887,7 +1886,7 @@ __device__ int wg_scan_incl(int v, int* wsum, int* total) {
   if (lane == 63) wsum[w] = v;
   __syncthreads();
   int add = 0, tot = 0;
-  for (int q = 0; q < (int)(blockDim.x >> 6); ++q) {
+  for (int q = 0; q < B / 64; ++q) {
     if (q < w) add += wsum[q];
     tot += wsum[q];
   }
@@ -1895,13 +1894,16 @@ __device__ int wg_scan_incl(int v, int* wsum, int* total) {
   *total = tot;
   return v + add;
 }
-// Per track: exclusive scans of the F1 face counts (slot offsets, owner of
-// each slot, the track's total) and of the fresh-source counts (down-slot
-// offsets), a workgroup's threads at a time; the next chunk's counts are loaded while the
-// current chunk is scanned.
-__device__ void wg_f1_scan(const Dev& d, int j) {
+// Per track: exclusive scan of the cells' upper-neighbour counts (F1 face slots'
+// offsets, owner of each slot, the track's total), a workgroup's threads at a
+// time; the next chunk's counts are loaded while the current chunk is scanned.
+// BT: the workgroup's threads where they are fixed (0: as launched), which
+// takes 0.1 us off a chunk of 256 cells (9 tracks of 128,000 cells 3042 -> 2831
+// us a step).
+template <int BT>
+__device__ __forceinline__ void wg_f1_scan(const Dev& d, int j) {
   __shared__ int wsum[KB / 64];
-  int B = (int)blockDim.x;
+  const int B = BT ? BT : (int)blockDim.x;
   int nt = d.ntrack[j];
   const int* cnt = d.nbucnt;
   int base = 0;
@@ -1911,7 +1913,7 @@ __device__ void wg_f1_scan(const Dev& d, int j) {
     int v = vnext < 0 ? 0 : vnext;
     vnext = i + B < nt ? cnt[CI(d, j, i + B)] : 0;
     int tot;
-    int off = base + wg_scan_incl(v, wsum, &tot) - v;
+    int off = base + wg_scan_incl(v, wsum, &tot, B) - v;
     if (i < nt) {
       d.f1off[CI(d, j, i)] = off;
       for (int n = 0; n < v && off + n < d.fcap; ++n) d.f1own[(long long)j * d.fcap + off + n] = i;
@@ -1923,7 +1925,7 @@ __device__ void wg_f1_scan(const Dev& d, int j) {
     if (base > d.fcap) atomicAdd(cnt_at(d, CNT_F1OVF), 1ull);
   }
 }
-__global__ void __launch_bounds__(KB) k_f1_scan(Dev d) { wg_f1_scan(d, (int)blockIdx.x); }
+__global__ void __launch_bounds__(KB) k_f1_scan(Dev d) { wg_f1_scan<KB>(d, (int)blockIdx.x); }
 // cell pass with the gradient cache in LDS: thread t's entry m at
 // cache[m * blockDim + t] (consecutive lanes, consecutive banks); the launch
 // passes blockDim * f1_kc * NQ doubles of dynamic LDS.  The pass waits on
@@ -1941,7 +1943,7 @@ k_f1grad(Dev d, int ni, int remap, int y0) {
     // 2 to 4 % of a step on grids to 512 x 512, 0.5 % on the largest)
     if ((int)blockIdx.y < y0) {
       int j = (int)(blockIdx.y * gridDim.x + blockIdx.x);
-      if (j < d.nj) wg_f1_scan(d, j);
+      if (j < d.nj) wg_f1_scan<0>(d, j);
       return;
     }
     int i, j;
@@ -2964,6 +2966,7 @@ struct gammahip_ctx {
   int block = 128;         // threads per workgroup of the per-cell kernels (64..256)
   bool block_auto = true;  // block follows BLOCK64_LIVE until the option sets it (2D)
   long long live = 0;      // wavefronts of 64 live cells at load
+  int longest = 0;         // cells of the longest track at load
   bool f1fuse_auto = true; // F1 sums in the update by f1_sums_in_update until the option says so
   int remap = 2;           // tile order: 0 hardware, 1 XCD bands, 2 track groups
   int use_graph = 0;       // replay steps from a captured hipGraph
@@ -2994,6 +2997,18 @@ struct gammahip_ctx {
 };
 
 namespace {
+
+// The scan of a track's F1 face slots takes its cells a workgroup's threads at
+// a time, one chunk after the other, so it rides with the gradients only while
+// they last longer: with six fields up to 16 chunks, with ten 96, and one more
+// per 110 live wavefronts.  Riding against a launch of its own (256 threads), us
+// a step: 9 tracks of 1000 cells 189 / 197, 2000 232 / 216, 16000 601 / 494; 32
+// of 1000 216 / 225, 6000 444 / 445, 16000 886 / 830; 128 of 2000 437 / 462,
+// 16000 2231 / 2345; 1024 of 4000 4181 / 4217; jets of 12 tracks to 3900 cells
+// 376 / 386, 512 to 3900 2074 / 2124, 5 to 3300 1333 / 1358, 5 to 6500 2694 / 2678.
+bool scan_rides(const gammahip_ctx* c) {
+  return (c->longest + c->block - 1) / c->block <= (c->cfg.nq == 10 ? 96 : 16) + c->live / 110;
+}
 
 int fail(gammahip_ctx* c, const std::string& m) {
   if (c) c->err = m;
@@ -3277,7 +3292,7 @@ struct Pipe {
       }
 #else
       // the scan rides with the gradient pass, where its rows fit the grid
-      bool grad_scan = !d.packed && !nbgrad && !c->f1cell && !d.pc && d.nj <= 32767;
+      bool grad_scan = !d.packed && !nbgrad && !c->f1cell && !d.pc && d.nj <= 32767 && scan_rides(c);
       if (!grad_scan) hipLaunchKernelGGL(k_f1_scan, dim3(d.nj), dim3(KB), 0, c->stream, d);
 #endif
       if (c->f1cell) {
@@ -3960,8 +3975,9 @@ int gammahip_load(gammahip_ctx* c, const double* x, const double* dx, const doub
   }
   c->live = 0;
   for (int j = 0; j < nj; ++j) c->live += (ntrack[j] + 63) / 64;
+  c->longest = *std::max_element(ntrack.begin(), ntrack.end());
   d.rgch = 0;
-  if (rg_screen_chipwide(d.rg_mode, nj, *std::max_element(ntrack.begin(), ntrack.end()))) {
+  if (rg_screen_chipwide(d.rg_mode, nj, c->longest)) {
     long long units = (d.nax + RGS - 1) / RGS;           // about 1024 workgroups: four a CU
     d.rgspan = RGS * (int)(1 + nj * units / 1024);
     d.rgch = (d.nax + d.rgspan - 1) / d.rgspan;

@@ -50,3 +50,15 @@ def test_gpu_regrid_other_rules(case):
         if case == "expanding_circ":
             s = dataclasses.replace(s, cfg=s.cfg.replace(circ_regrid=1))
     _equal(s, (1, 35) if case == "riemann" else (1, 9))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1200, 1300, 1700])
+def test_gpu_slot_scan_with_and_without_the_gradients(n):
+    """Track lengths on either side of where the F1 slot scan gets a launch of its own."""
+    s = S.riemann_2d(n, 9, ly=9 / n)
+    g, o = hip.Grid(s), oc.OracleGrid(s)
+    g.step(12)
+    o.run(12)
+    for f in (S.RHO, S.PPP, S.UU1, S.UU2, hip.F_X):
+        assert np.array_equal(np.concatenate(g.active(f)), np.concatenate(o.active(f))), f
