@@ -65,6 +65,12 @@ constexpr int DT_CH = 1024;   // cells per workgroup of the per-track dt minimum
 // most CUs (24 tracks of 512-2048 cells 135 us a step, against 165 and 138 with
 // 128 and 256 threads; 256 tracks 770 against 804 and 809).
 constexpr int S1B = 64, S1C = S1B - 1;
+// Cells of the longest track at load from which the tiles' dt minima are reduced
+// in a launch (k1_dt_min) instead of by every wavefront of the first stage,
+// which grows with the square of the length.  Wavefronts against launch, us a
+// step: one track of 16,000 cells 70.4 / 70.9, 64,000 77.9 / 76.5, 256,000
+// 115 / 103, a million 539 / 329; 64 tracks of 16,000 303 / 304, 40,000 775 / 757.
+constexpr int S1MIN_FROM = 512 * S1C;
 
 // ---------------------------------------------------------------------------
 // device view (passed by value to every kernel)
@@ -89,6 +95,7 @@ struct Dev {
   int* rgpart;             // [nj][rgch][3] what k_rg_screen found: last cell past the shock threshold, first and last flagged
   int rgch, rgspan;        // k_rg_screen: workgroups per track (0: k_regrid screens its track itself), slots of each
   int dtch;                // chunks per track: ceil(nax / DT_CH)
+  int s1min;               // 1D: the tracks' dt minima come from k1_dt_min
   int s1ch;                // 1D: tiles per track of the stage passes, ceil(nax / S1C); tpart is [nj][s1ch] there
   // cells
   double *primn, *cxn, *cdxn;   // 1D: the stage passes' output state (swapped with prim, cx, cdx)
@@ -2495,6 +2502,20 @@ __global__ void __launch_bounds__(S1B) k1_faces(Dev d) {
     d.tpart[(long long)j * d.s1ch + blockIdx.x] = m;
   }
 }
+// the minimum of each track's tiles, ahead of the first stage, where there are
+// too many for every wavefront of the stage to read
+__global__ void __launch_bounds__(1024) k1_dt_min(Dev d) {
+  __shared__ double sm[16];
+  int j = (int)blockIdx.x, t = (int)threadIdx.x, n = (d.ntrack[j] + S1C - 1) / S1C;
+  double m = 1.e15;
+  for (int q = t; q < n; q += 1024) m = fmin(m, d.tpart[(long long)j * d.s1ch + q]);
+  for (int s = 32; s > 0; s >>= 1) m = fmin(m, __shfl_xor(m, s, 64));
+  if ((t & 63) == 0) sm[t >> 6] = m;
+  __syncthreads();
+  if (t) return;
+  for (int q = 1; q < 16; ++q) m = fmin(m, sm[q]);
+  d.tmin[j] = m;
+}
 template <int NQ, bool SHK, int SV, int STAGE, bool STD>
 __global__ void __launch_bounds__(S1B) k1_stage(Dev d) {
   s1_options(d, STD);
@@ -2506,13 +2527,18 @@ __global__ void __launch_bounds__(S1B) k1_stage(Dev d) {
   double dt;
   if (STAGE == 1) {
     // the track's minimum over its tiles, by every wavefront for itself (a
-    // minimum does not depend on the order it is taken in)
+    // minimum does not depend on the order it is taken in), or k1_dt_min's
     double m = 1.e15;
     int n = (nt + S1C - 1) / S1C;
-    for (int q = t & 63; q < n; q += 64) m = fmin(m, d.tpart[(long long)j * d.s1ch + q]);
-    for (int s = 32; s > 0; s >>= 1) m = fmin(m, __shfl_xor(m, s, 64));
+    if (d.s1min) m = d.tmin[j];
+    else for (int q = t & 63; q < n; q += 64) m = fmin(m, d.tpart[(long long)j * d.s1ch + q]);
+    if (!d.s1min)
+      for (int s = 32; s > 0; s >>= 1) m = fmin(m, __shfl_xor(m, s, 64));
     dt = d.P.cfl * m;
-    if (blockIdx.x == 0 && t == 0) { d.tmin[j] = m; d.tdt[j] = dt; }
+    if (blockIdx.x == 0 && t == 0) {
+      if (!d.s1min) d.tmin[j] = m;
+      d.tdt[j] = dt;
+    }
   } else {
     dt = d.tdt[j];
   }
@@ -3548,6 +3574,7 @@ struct Pipe {
     bool std = !d.P.synge && !d.pc && !d.vpspec;
     if (std) hipLaunchKernelGGL((k1_faces<NQ, SHK, true>), tiles, dim3(S1B), 0, c->stream, d);
     else hipLaunchKernelGGL((k1_faces<NQ, SHK, false>), tiles, dim3(S1B), 0, c->stream, d);
+    if (d.s1min) hipLaunchKernelGGL(k1_dt_min, dim3(d.nj), dim3(1024), 0, c->stream, d);
     auto stage = [&](auto st, auto sv) {
       constexpr int ST = decltype(st)::value, SV = decltype(sv)::value;
       if (std) hipLaunchKernelGGL((k1_stage<NQ, SHK, SV, ST, true>), tiles, dim3(S1B), 0, c->stream, d);
@@ -3976,6 +4003,7 @@ int gammahip_load(gammahip_ctx* c, const double* x, const double* dx, const doub
   c->live = 0;
   for (int j = 0; j < nj; ++j) c->live += (ntrack[j] + 63) / 64;
   c->longest = *std::max_element(ntrack.begin(), ntrack.end());
+  d.s1min = c->longest > S1MIN_FROM;
   d.rgch = 0;
   if (rg_screen_chipwide(d.rg_mode, nj, c->longest)) {
     long long units = (d.nax + RGS - 1) / RGS;           // about 1024 workgroups: four a CU

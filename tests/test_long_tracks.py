@@ -62,3 +62,16 @@ def test_gpu_slot_scan_with_and_without_the_gradients(n):
     o.run(12)
     for f in (S.RHO, S.PPP, S.UU1, S.UU2, hip.F_X):
         assert np.array_equal(np.concatenate(g.active(f)), np.concatenate(o.active(f))), f
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [32_252, 32_253, 64_000])
+def test_gpu_1d_time_step_of_many_tiles(n):
+    """Track lengths (four ghost cells more) on either side of where the tiles' minima get a launch of their own."""
+    s = S.shock_tube_1d(n)
+    g, o = hip.Grid(s), oc.OracleGrid(s)
+    g.step(5)
+    o.run(5)
+    for f in (S.RHO, S.PPP, S.UU1, hip.F_X):
+        assert np.array_equal(g.active(f)[0], o.active(f)[0]), f
+    assert g.time()[0][0] == o.t
