@@ -2470,6 +2470,14 @@ __global__ void __launch_bounds__(RG ? RGB : 64) k1_begin(Dev d) {
   }
   if ((int)threadIdx.x < 2 * d.ngst) body_ghost_mv<1, NQ>(d, j, (int)threadIdx.x);
 }
+// all slots past the tracks' ends into the second planes: restoring 64 tracks of
+// 512 to 4096 cells took 1185 us without a second set and 1277 with a copy of
+// each plane, and takes 1131 where it took 1139; one track of 4000 cells 18 us
+// more than without, the launch and its wait, which its first step gives back
+__global__ void __launch_bounds__(256) k1_mirror(Dev d, int ch) {
+  int j = (int)blockIdx.x / ch, i = ((int)blockIdx.x - j * ch) * 256 + (int)threadIdx.x;
+  if (i >= d.ntrack[j] && i < d.nax) mirror_slot(d, CI(d, j, i));
+}
 // STD: constant adiabatic index, piecewise-linear reconstruction, constant
 // spectral index -- the options that run-time switches otherwise keep apart in
 // these kernels, splitting their arithmetic into blocks the compiler cannot
@@ -3083,20 +3091,20 @@ int d2h(gammahip_ctx* c, void* dst, const void* src, size_t bytes) {
 #endif
 }
 
-// 1D: the stage passes' second planes take the values of the first (which hold
-// the state just loaded or restored)
+// 1D: slots past the tracks' ends take the same values in the stage passes'
+// second planes as in the first (which hold the state just loaded or restored);
+// the slots of live cells are written by the stage that first swaps them in
 int mirror_state(gammahip_ctx* c) {
   Dev& d = c->d;
   if (d.nd != 1) return 0;
-  std::pair<double*, double*> pl[3] = {{d.primn, d.prim}, {d.cxn, d.cx}, {d.cdxn, d.cdx}};
-  for (int q = 0; q < 3; ++q) {
-    size_t bytes = sizeof(double) * (size_t)d.cs * (q == 0 ? d.nqs : 1);
 #ifdef GH_EMU
-    memcpy(pl[q].first, pl[q].second, bytes);
+  for (int j = 0; j < d.nj; ++j)
+    for (int i = d.ntrack[j]; i < d.nax; ++i) mirror_slot(d, CI(d, j, i));
 #else
-    HIPCHK(hipMemcpyAsync(pl[q].first, pl[q].second, bytes, hipMemcpyDeviceToDevice, c->stream));
+  int ch = (d.nax + 255) / 256;
+  hipLaunchKernelGGL(k1_mirror, dim3(d.nj * ch), dim3(256), 0, c->stream, d, ch);
+  HIPCHK(hipGetLastError());
 #endif
-  }
   return 0;
 }
 
@@ -3886,7 +3894,10 @@ int gammahip_create(const gammahip_config* cfg, gammahip_ctx** out) {
   e |= dalloc(c, &d.fv, cs); e |= dalloc(c, &d.flL, cs); e |= dalloc(c, &d.flR, cs);
   e |= dalloc(c, &d.fflux, nqs * cs);
   e |= dalloc(c, &d.cnt, (size_t)CNT_N * CNT_PARTS); e |= dalloc(c, &d.nsplit, nj); e |= dalloc(c, &d.nmerge, nj);
-  if (d.nd == 1) { e |= dalloc(c, &d.primn, nqs * cs); e |= dalloc(c, &d.cxn, cs); e |= dalloc(c, &d.cdxn, cs); }
+  if (d.nd == 1) {                          // one allocation: primn, cxn, cdxn
+    e |= dalloc(c, &d.primn, (nqs + 2) * cs);
+    if (!e) { d.cxn = d.primn + nqs * cs; d.cdxn = d.cxn + cs; }
+  }
   if (d.nd == 2) {
     e |= dalloc(c, &d.gmv, nqs * cs); e |= dalloc(c, &d.gf1, nqs * cs); e |= dalloc(c, &d.gf1n, nqs * cs);
     e |= dalloc(c, &d.nbdj, cs); e |= dalloc(c, &d.nbdlo, cs); e |= dalloc(c, &d.nbdcnt, cs);
