@@ -1,15 +1,15 @@
 """Autotuner for the launch options of the HIP backend.
 
-Options: threads per workgroup of the per-cell kernels (64, 128, 256),
-XCD-aware tile order (off/on), two-step hipGraph replay (off/on), persistent
-packed launch (off, or at most 4, 8, 16 or 32 workgroups per CU, each
-kernel's grid capped at what its registers and LDS let a CU hold), the register-capped builds of
-the F1 face kernel and of the update kernel (bit set, 0-3), the F1 flux sums
-inside the update kernel (off/on), the fused F1 gradient-and-face pass
-(off/on), the cons2prim solver (Brent, the
-reference's algorithm, or Newton) and, when a trained network is given, the
-learned cons2prim start (off, or on with trigger exponents 2 and 4; Newton
-only).
+Options: threads per workgroup of the per-cell kernels (the library's choice
+for the grid, 64, 128, 256), XCD-aware tile order (off/on), two-step hipGraph
+replay (off/on), persistent packed launch (off, or at most 4, 8, 16 or 32
+workgroups per CU, each kernel's grid capped at what its registers and LDS let
+a CU hold), the register-capped builds of the F1 face kernel and of the update
+kernel (bit set, 0-3), the F1 flux sums inside the update kernel (the library's
+choice, off, on), the fused F1 gradient-and-face pass (off/on), the cons2prim
+solver (Brent, the reference's algorithm, or Newton) and, when a trained network
+is given, the learned cons2prim start (off, or on with trigger exponents 2 and
+4; Newton only).
 
 Search: coordinate descent from the defaults -- each option in turn is set to
 each of its values with the others held, the fastest kept -- repeated for
@@ -24,9 +24,9 @@ from __future__ import annotations
 
 import time
 
-SPACE = (("solver", (0, 1)), ("block", (64, 128, 256)), ("remap", (0, 1, 2)), ("graph", (0, 1)),
-         ("persist", (0, 4, 8, 16, 32)), ("occ", (0, 1, 2, 3)), ("f1fuse", (0, 1)), ("f1cell", (0, 1)), ("fuse", (0, 1, 2, 4)))
-DEFAULTS = {"solver": 1, "block": 128, "remap": 2, "graph": 0, "persist": 0, "occ": 0, "f1fuse": 0,
+SPACE = (("solver", (0, 1)), ("block", ("auto", 64, 128, 256)), ("remap", (0, 1, 2)), ("graph", (0, 1)),
+         ("persist", (0, 4, 8, 16, 32)), ("occ", (0, 1, 2, 3)), ("f1fuse", ("auto", 0, 1)), ("f1cell", (0, 1)), ("fuse", (0, 1, 2, 4)))
+DEFAULTS = {"solver": 1, "block": "auto", "remap": 2, "graph": 0, "persist": 0, "occ": 0, "f1fuse": "auto",
             "f1cell": 0, "fuse": 0, "mlp_thr": None}
 OPTION_KEYS = tuple(DEFAULTS)
 # the plain form: the library's default launch with the reference's Brent solver

@@ -2998,7 +2998,7 @@ struct gammahip_ctx {
   // 2 % faster); the XCD bands help the uniform grid a little more but cost
   // the uneven ones up to 2x
   int block = 128;         // threads per workgroup of the per-cell kernels (64..256)
-  bool block_auto = true;  // block follows BLOCK64_LIVE until the option sets it (2D)
+  bool block_auto = true;  // block follows BLOCK64_LIVE (2D) until the option sets it
   long long live = 0;      // wavefronts of 64 live cells at load
   int longest = 0;         // cells of the longest track at load
   bool f1fuse_auto = true; // F1 sums in the update by f1_sums_in_update until the option says so
@@ -3031,6 +3031,13 @@ struct gammahip_ctx {
 };
 
 namespace {
+
+// options left to the rules, from the live cells at load
+void auto_rules(gammahip_ctx* c) {
+  bool two = c->cfg.nd == 2;
+  if (c->block_auto) c->block = two && c->live <= BLOCK64_LIVE ? 64 : 128;
+  if (c->f1fuse_auto) c->d.f1fused = two && f1_sums_in_update(c->cfg.nq, c->live) ? 1 : 0;
+}
 
 // The scan of a track's F1 face slots takes its cells a workgroup's threads at
 // a time, one chunk after the other, so it rides with the gradients only while
@@ -4021,8 +4028,7 @@ int gammahip_load(gammahip_ctx* c, const double* x, const double* dx, const doub
     d.rgspan = RGS * (int)(1 + nj * units / 1024);
     d.rgch = (d.nax + d.rgspan - 1) / d.rgspan;
   }
-  if (cf.nd == 2 && c->f1fuse_auto) d.f1fused = f1_sums_in_update(cf.nq, c->live) ? 1 : 0;
-  if (cf.nd == 2 && c->block_auto) c->block = c->live <= BLOCK64_LIVE ? 64 : 128;
+  auto_rules(c);
   int e = 0;
   e |= h2d(c, d.ntrack, ntrack.data(), sizeof(int) * nj);
   e |= h2d(c, d.trg, trg.data(), sizeof(int) * nj);
@@ -4116,6 +4122,13 @@ int gammahip_set_option(gammahip_ctx* c, int key, long long value) {
       build_tiles(c);
       return post(c);
     case GAMMAHIP_OPT_F1FUSE: c->d.f1fused = value ? 1 : 0; c->f1fuse_auto = false; return 0;
+    case GAMMAHIP_OPT_AUTO:
+      if (value < 0 || value > 3) return fail(c, "automatic options must be a bit set in 0..3");
+      if (value & 1) c->block_auto = true;
+      if (value & 2) c->f1fuse_auto = true;
+      auto_rules(c);
+      build_tiles(c);
+      return post(c);
     case GAMMAHIP_OPT_F1CELL: c->f1cell = value ? 1 : 0; return 0;
     case GAMMAHIP_OPT_FUSE:
       if (value < 0 || value > 7) return fail(c, "fuse option must be in 0..7");

@@ -24,7 +24,7 @@ F_GRADMV0, F_GRADF10 = 300, 400
 FACE_X, FACE_V, FACE_LL, FACE_LR, FACE_FLUX0 = 1000, 1001, 1002, 1003, 1010
 RESET_SHOCK, DETECT_SHOCK, INJECT, INIT_GAMMAS, ADVANCE_TIME = range(5)
 C2P_BRENT, C2P_NEWTON = 0, 1
-OPT_BLOCK, OPT_REMAP, OPT_GRAPH, OPT_MLP_THR, OPT_PERSIST, OPT_OCC, OPT_F1FUSE, OPT_SOLVER, OPT_F1CELL, OPT_FUSE, OPT_USER_CELL = range(11)
+OPT_BLOCK, OPT_REMAP, OPT_GRAPH, OPT_MLP_THR, OPT_PERSIST, OPT_OCC, OPT_F1FUSE, OPT_SOLVER, OPT_F1CELL, OPT_FUSE, OPT_USER_CELL, OPT_AUTO = range(12)
 
 
 class Config(C.Structure):
@@ -260,7 +260,13 @@ class Grid:
         transverse-gradient and own-face F1 pass; fused passes (bit 0: the F1
         neighbour search inside the transverse-gradient pass; bit 1: MV
         gradients recomputed in the F1 passes; bit 2: F1 faces one thread per
-        owner cell)."""
+        owner cell).  block and f1fuse may be "auto": the library's own choice
+        for this grid, which holds until either is set."""
+        auto = (block == "auto") + 2 * (f1fuse == "auto")
+        if auto:
+            self._check(self.L.gammahip_set_option(self.h, OPT_AUTO, auto))
+            block = None if block == "auto" else block
+            f1fuse = None if f1fuse == "auto" else f1fuse
         for key, val in ((OPT_SOLVER, solver), (OPT_BLOCK, block), (OPT_REMAP, remap), (OPT_GRAPH, graph),
                          (OPT_MLP_THR, mlp_thr), (OPT_PERSIST, persist), (OPT_OCC, occ),
                          (OPT_F1FUSE, f1fuse), (OPT_F1CELL, f1cell), (OPT_FUSE, fuse)):

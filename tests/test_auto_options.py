@@ -1,0 +1,54 @@
+"""The options that the library chooses by the grid (workgroup size, F1 sums
+inside the update) can be given back to it, and the tuner starts from, compares
+with and falls back to that choice."""
+from __future__ import annotations
+
+import pytest
+
+from gamma_amd import autotune, hip, setups as S
+
+
+class _Recorder:
+    """A grid that notes the options set on it."""
+
+    def __init__(self):
+        self.opts = {}
+
+    def set_options(self, **kw):
+        self.opts.update(kw)
+
+    def load_surrogate(self, w):
+        pass
+
+
+@pytest.mark.parametrize("form", ["DEFAULTS", "PLAIN"])
+def test_tuner_starts_from_the_librarys_choice(form):
+    g = _Recorder()
+    autotune.apply(g, getattr(autotune, form))
+    assert g.opts["block"] == "auto" and g.opts["f1fuse"] == "auto"
+    space = dict(autotune.SPACE)
+    assert "auto" in space["block"] and "auto" in space["f1fuse"]
+
+
+def test_emu_auto_value_is_taken_and_checked(emu_lib):
+    g = hip.Grid(S.riemann_2d(32, 8), lib_path=emu_lib)
+    g.set_options(block=256, f1fuse=1)
+    g.set_options(block="auto", f1fuse="auto")
+    for bad in (-1, 4):
+        assert g.L.gammahip_set_option(g.h, hip.OPT_AUTO, bad) != 0
+    with pytest.raises(RuntimeError, match="block"):
+        g.set_options(block=96)
+
+
+@pytest.mark.gpu
+def test_gpu_f1_sums_return_to_the_rule():
+    """Ten fields: summed in the update unless asked otherwise (entry 4 of the
+    kernel times counts the separate pass)."""
+    g = hip.Grid(S.bm_jet_2d(12, 0.3, 40, 160))
+    g.kernel_times()
+    seen = []
+    for opt in (None, 0, "auto", 1, "auto"):
+        g.set_options(f1fuse=opt)
+        g.step(2)
+        seen.append(int(g.kernel_times()[1][4]))
+    assert seen == [0, 6, 0, 0, 0]
