@@ -3,9 +3,11 @@ inside the update) can be given back to it, and the tuner starts from, compares
 with and falls back to that choice."""
 from __future__ import annotations
 
+import numpy as np
 import pytest
 
 from gamma_amd import autotune, hip, setups as S
+import oracle_ctypes as oc
 
 
 class _Recorder:
@@ -52,3 +54,22 @@ def test_gpu_f1_sums_return_to_the_rule():
         g.step(2)
         seen.append(int(g.kernel_times()[1][4]))
     assert seen == [0, 6, 0, 0, 0]
+
+
+def _separate_sums(lib_path):
+    s = S.bm_jet_2d(12, 0.3, 40, 160)
+    g, o = hip.Grid(s, lib_path=lib_path), oc.OracleGrid(s)
+    g.set_options(block=128, f1fuse=0)
+    g.step(30)
+    o.run(30)
+    for f in (S.RHO, S.PPP, S.UU1, S.UU2, S.GMX, hip.F_X):
+        assert all(np.array_equal(a, b) for a, b in zip(g.active(f), o.active(f))), f
+
+
+def test_emu_ten_fields_with_the_sums_in_a_pass_of_their_own(emu_lib):
+    _separate_sums(emu_lib)
+
+
+@pytest.mark.gpu
+def test_gpu_ten_fields_with_the_sums_in_a_pass_of_their_own():
+    _separate_sums(hip.LIB_PATH)
