@@ -3533,11 +3533,11 @@ struct Pipe {
     ghosts(c); prep(c, false); update(c, 3 | tail);
   }
   // the 1D step in five passes; general otherwise: packed launches, the learned
-  // start, Euler steps, event timing of the separate passes, and user hooks
-  // that read the track's time while a stage runs
+  // start, Euler steps, and user hooks that read the track's time while a stage
+  // runs
   static bool fused1(const gammahip_ctx* c) {
     const Dev& d = c->d;
-    return ND == 1 && !d.packed && !d.mw && !d.euler && !d.ucell && !c->timing && !c->user_hooks &&
+    return ND == 1 && !d.packed && !d.mw && !d.euler && !d.ucell && !c->user_hooks &&
            d.nj <= 65535;               // tracks are the grid's second dimension
   }
   template <bool SHK>
@@ -3587,13 +3587,17 @@ struct Pipe {
     if (d.rg_mode) hipLaunchKernelGGL((k1_begin<NQ, true>), dim3(d.nj), dim3(RGB), 0, c->stream, d);
     else hipLaunchKernelGGL((k1_begin<NQ, false>), dim3(d.nj), dim3(64), 0, c->stream, d);
     bool std = !d.P.synge && !d.pc && !d.vpspec;
+    tbeg(c, 1);
     if (std) hipLaunchKernelGGL((k1_faces<NQ, SHK, true>), tiles, dim3(S1B), 0, c->stream, d);
     else hipLaunchKernelGGL((k1_faces<NQ, SHK, false>), tiles, dim3(S1B), 0, c->stream, d);
+    tend(c, 1);
     if (d.s1min) hipLaunchKernelGGL(k1_dt_min, dim3(d.nj), dim3(1024), 0, c->stream, d);
     auto stage = [&](auto st, auto sv) {
       constexpr int ST = decltype(st)::value, SV = decltype(sv)::value;
+      tbeg(c, 0);
       if (std) hipLaunchKernelGGL((k1_stage<NQ, SHK, SV, ST, true>), tiles, dim3(S1B), 0, c->stream, d);
       else hipLaunchKernelGGL((k1_stage<NQ, SHK, SV, ST, false>), tiles, dim3(S1B), 0, c->stream, d);
+      tend(c, 0);
       swap();
     };
 #endif

@@ -171,8 +171,12 @@ int  gammahip_stats_get(gammahip_ctx* ctx, gammahip_stats* st);
 int  gammahip_regrid_counts(gammahip_ctx* ctx, long long* splits, long long* merges);
 /* Average duration (ms) of the dominant kernel launches since the last call,
  * measured with HIP events on the context's stream: entry 0 the update, 1 the
- * MV face pass (small 2D grids: with the F1 neighbour search), 2 the F1 face pass, 3 the transverse-gradient pass, 4 the F1
- * flux sums, 5 the fused gradient-and-face pass. */
+ * MV face pass (small 2D grids: with the F1 neighbour search), 2 the F1 face
+ * pass, 3 the transverse-gradient pass, 4 the F1 flux sums, 5 the fused
+ * gradient-and-face pass.  The five-launch step of 1D grids: entry 0 the three
+ * stage passes (the second and third with their faces), 1 the first face pass.
+ * The first call switches the events on for the context's life; steps then take
+ * the same launches as before it, but are not replayed from a graph. */
 int  gammahip_kernel_times(gammahip_ctx* ctx, double* ms_per_launch /* [16] */,
                            long long* launches /* [16] */);
 int  gammahip_sync(gammahip_ctx* ctx);
