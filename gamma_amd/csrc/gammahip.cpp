@@ -3799,6 +3799,7 @@ int run_batch(long long n, BatchArrays in, BatchArrays out, Launch&& launch) {
       if (row == a.bytes) {
         memcpy(h, src, (size_t)m * row);
       } else {                          // rows of three doubles out of longer ones
+        if (a.bytes != 24 || row < 24) return plain_fail("batch rows: only three doubles of longer rows are packed");
         for (long long q = 0; q < m; ++q) memcpy(h + (size_t)q * 24, src + (size_t)q * row, 24);
       }
       ptr[np++] = S.s[k].d + at;
