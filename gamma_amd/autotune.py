@@ -13,7 +13,7 @@ is given, the learned cons2prim start (off, or on with trigger exponents 2 and
 
 Search: coordinate descent from the defaults -- each option in turn is set to
 each of its values with the others held, the fastest kept -- repeated for
-`sweeps` passes.  Each evaluation runs on the live grid (the production state,
+`sweeps` passes; options without effect on the grid (no_effect) are left out.  Each evaluation runs on the live grid (the production state,
 not a toy): a short untimed run to settle (and capture the graph), then
 `steps` timed steps between stream synchronisations.  The grid keeps evolving
 while tuning, so the incumbent is re-timed with every challenger and the
@@ -24,6 +24,8 @@ from __future__ import annotations
 
 import time
 
+from . import setups as S
+
 SPACE = (("solver", (0, 1)), ("block", ("auto", 64, 128, 256)), ("remap", (0, 1, 2)), ("graph", (0, 1)),
          ("persist", (0, 4, 8, 16, 32)), ("occ", (0, 1, 2, 3)), ("f1fuse", ("auto", 0, 1)), ("f1cell", (0, 1)), ("fuse", (0, 1, 2, 4)))
 DEFAULTS = {"solver": 1, "block": "auto", "remap": 2, "graph": 0, "persist": 0, "occ": 0, "f1fuse": "auto",
@@ -31,6 +33,24 @@ DEFAULTS = {"solver": 1, "block": "auto", "remap": 2, "graph": 0, "persist": 0, 
 OPTION_KEYS = tuple(DEFAULTS)
 # the plain form: the library's default launch with the reference's Brent solver
 PLAIN = dict(DEFAULTS, solver=0)
+
+
+def no_effect(grid, key: str, cand: dict) -> bool:
+    """Whether an option changes nothing on this grid with the others as in
+    cand: in 1D there are no F1 passes, and the five-launch step (all but
+    packed launches, the learned start, Euler steps and user hooks) has launches
+    of its own."""
+    rc = grid.rc
+    if rc.nd != 1:
+        return False
+    if key in ("f1fuse", "f1cell", "fuse"):
+        return True
+    if key not in ("block", "remap", "occ"):
+        return False
+    hooks = [h for h in grid.setup.hooks or [] if h]
+    user = any(S.KIN_USER == h.get("kin_mode", rc.kin_mode) or S.BND_USER == h.get("bnd_mode", rc.bnd_mode)
+               for h in hooks + [{}])
+    return not (cand["persist"] or cand["mlp_thr"] is not None or rc.timestep == S.TS_EULER or rc.user_cell or user)
 
 
 def apply(grid, cand: dict, surrogate=None):
@@ -62,7 +82,7 @@ def tune(grid, steps: int = 6, settle: int = 2, sweeps: int = 2, surrogate=None,
     for _ in range(sweeps):
         for key, values in space:
             for v in values:
-                if v == best[key]:
+                if v == best[key] or no_effect(grid, key, best):
                     continue
                 cand = dict(best, **{key: v})
                 if cand["mlp_thr"] is not None and cand["solver"] != 1:

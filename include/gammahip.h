@@ -205,7 +205,10 @@ int  gammahip_sync(gammahip_ctx* ctx);
  * Brent (0, the reference's algorithm) and Newton (1; required while the
  * learned guess is loaded); F1CELL 1 computes each cell's transverse gradient
  * and then the fluxes of its own F1 faces in one pass, the owner's state kept
- * in registers, instead of a gradient pass and a one-thread-per-face pass. */
+ * in registers, instead of a gradient pass and a one-thread-per-face pass.
+ * 1D grids: F1FUSE, F1CELL and FUSE change nothing, and BLOCK, REMAP and OCC only
+ * the general passes (packed launches, the learned start, Euler steps, user
+ * hooks); the five-launch step has launches of its own. */
 enum { GAMMAHIP_OPT_BLOCK = 0, GAMMAHIP_OPT_REMAP = 1, GAMMAHIP_OPT_GRAPH = 2,
        GAMMAHIP_OPT_MLP_THR = 3, GAMMAHIP_OPT_PERSIST = 4, GAMMAHIP_OPT_OCC = 5,
        GAMMAHIP_OPT_F1FUSE = 6, GAMMAHIP_OPT_SOLVER = 7, GAMMAHIP_OPT_F1CELL = 8,

@@ -73,3 +73,27 @@ def test_emu_ten_fields_with_the_sums_in_a_pass_of_their_own(emu_lib):
 @pytest.mark.gpu
 def test_gpu_ten_fields_with_the_sums_in_a_pass_of_their_own():
     _separate_sums(hip.LIB_PATH)
+
+
+@pytest.mark.parametrize("setup,cand,idle", [
+    (lambda: S.shock_tube_1d(32), {}, {"block", "remap", "occ", "f1fuse", "f1cell", "fuse"}),
+    (lambda: S.shock_tube_1d(32), {"persist": 8}, {"f1fuse", "f1cell", "fuse"}),
+    (lambda: S.shock_tube_1d(32), {"mlp_thr": 2}, {"f1fuse", "f1cell", "fuse"}),
+    (lambda: S.reflecting_box(32), {}, {"f1fuse", "f1cell", "fuse"}),
+    (lambda: S.ensemble_1d(4, sizes=(60, 80))[0], {}, {"block", "remap", "occ", "f1fuse", "f1cell", "fuse"}),
+    (lambda: S.riemann_2d(32, 8), {}, set()),
+])
+def test_emu_tuner_leaves_out_options_without_effect(emu_lib, setup, cand, idle):
+    g = hip.Grid(setup(), lib_path=emu_lib)
+    cand = dict(autotune.PLAIN, **cand)
+    assert {k for k, _ in autotune.SPACE if autotune.no_effect(g, k, cand)} == idle
+
+
+def test_emu_tuner_times_nothing_without_effect(emu_lib):
+    g = hip.Grid(S.shock_tube_1d(32), lib_path=emu_lib)
+    r = autotune.tune(g, steps=1, settle=1, sweeps=1)
+    for row in r["table"]:
+        plain = row["persist"] == 0
+        assert row["f1fuse"] == "auto" and row["f1cell"] == 0 and row["fuse"] == 0
+        assert not plain or (row["block"] == "auto" and row["remap"] == 2 and row["occ"] == 0)
+    assert {k: r["best"][k] for k in autotune.OPTION_KEYS}.keys() == autotune.DEFAULTS.keys()
