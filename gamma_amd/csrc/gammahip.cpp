@@ -3955,7 +3955,7 @@ int gammahip_load(gammahip_ctx* c, const double* x, const double* dx, const doub
   int nj = d.nj, nax = d.nax, ng = d.ngst, nm = cf.ncell_mv, na = cf.ntracks_active;
   size_t cs = d.cs;
   drop_graph(c);            // the rules below pick launches by the tracks' hooks and lengths
-  c->user_hooks = false;
+  bool user_hooks = false;  // the context's only once every track has been accepted
   // host images of the initial state (Cinit + mpi_distribute, 1d.cpp:956-969, 2d.cpp:1175-1195)
   std::vector<int> ntrack(nj, nm + 2 * ng), tgeom(nj), tkin(nj), tbnd(nj), trg(nj, RG_NONE);
   std::vector<double> tvin(nj), tvout(nj), tbm(4 * nj), ty(nj), tdy(nj), tt(nj, t0);
@@ -3973,7 +3973,7 @@ int gammahip_load(gammahip_ctx* c, const double* x, const double* dx, const doub
     trg[j] = h.rg_mode >= 0 ? h.rg_mode : cf.rg_mode;
     d.rg_mode |= trg[j] != RG_NONE ? (1 << trg[j]) : 0;
     tgeom[j] = cf.geom >= 0 ? cf.geom : h.geom;
-    c->user_hooks |= h.kin_mode == KIN_USER || h.bnd_mode == BND_USER;
+    user_hooks |= h.kin_mode == KIN_USER || h.bnd_mode == BND_USER;
     tkin[j] = h.kin_mode; tvin[j] = h.v_in; tvout[j] = h.v_out; tbnd[j] = h.bnd_mode;
     for (int q = 0; q < 4; ++q) tbm[4 * j + q] = h.bm[q];
     ty[j] = cf.nd == 2 ? y[a] : 0.;
@@ -4023,6 +4023,7 @@ int gammahip_load(gammahip_ctx* c, const double* x, const double* dx, const doub
       else hfx[k] = hx[k + 1] - hdx[k + 1] / 2.;
     }
   }
+  c->user_hooks = user_hooks;
   c->live = 0;
   for (int j = 0; j < nj; ++j) c->live += (ntrack[j] + 63) / 64;
   c->longest = *std::max_element(ntrack.begin(), ntrack.end());
