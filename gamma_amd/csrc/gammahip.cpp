@@ -221,9 +221,10 @@ GH_HD bool active_track(const Dev& d, int j) { return d.nd == 1 || (j > d.jL && 
 // copy every persistent per-cell field of (js,is) into (j,i).  All fields are
 // read before the first is written: the planes may alias for all the compiler
 // knows, so a field-by-field copy waits for each load before it issues the
-// next, up to 35 round trips to memory one after the other: a 2D grid's ghost
-// pass took 15.8 us with six fields (96 x 33) and 25.9 us with ten (48 uneven
-// tracks), and takes about 5.5 and 10 us with the reads together.
+// next, up to 42 round trips to memory one after the other (two dimensions, ten
+// fields, shock state): a 2D grid's ghost pass took 15.8 us with six fields
+// (96 x 33) and 25.9 us with ten (48 uneven tracks), and takes about 5.5 and 10 us
+// with the reads together.
 template <int ND, int NQ>
 GH_HD void copy_cell(const Dev& d, long long kd, long long ks) {
   constexpr int NS = ND == 1 ? NQ - 1 : NQ, NG = ND == 2 ? NS : 1;
@@ -556,7 +557,7 @@ GH_HD void trans_grad(const Dev& d, int j, long long k, const double* p0, const 
   for (int q = 0; q < NQ; ++q) gavg[q] = 0.;
   double dAtot = 0;
   // both lists at once: read where a side's loop begins, each cost a round trip
-  // of its own (2048^2 4330 -> 4210 us a step, 1024-track jet 4120 -> 4045)
+  // of its own (2048^2 4330 -> 4180 us a step, 1024-track jet 4115 -> 4040)
   const int tj0 = d.nbdj[k], lo0 = d.nbdlo[k], cn0 = d.nbdcnt[k], tj1 = d.nbuj[k], lo1 = d.nbulo[k], cn1 = d.nbucnt[k];
   for (int pass = 0; pass < 2; ++pass) {
     int idx = 0;
@@ -1084,8 +1085,9 @@ GH_HD void body_update(const Dev& d, int j, int i, int stage) {
 // in place of one launch per sweep (13 to 19 a step, of 4.5 us at least; a step
 // of a 64-cell track 93 -> 71 us, 4000 cells with particles 180 -> 128, 24
 // tracks 229 -> 135, 256 tracks 939 -> 770).  Small tracks are bound by the
-// latency of a cell's two root searches, the ensemble by FP64 issue (some 5900
-// vector instructions per wavefront and stage).  A stage reads the state
+// latency of a cell's two root searches, the ensemble by FP64 issue (97 M vector
+// instructions in a launch of its second or third stage, two thirds of the issue
+// slots while it runs).  A stage reads the state
 // of cells its workgroup does not own, so it writes to a second set of planes
 // (primn, cxn, cdxn, fxn) that the driver swaps in.  Same arithmetic in the
 // same order as the separate sweeps.  Fluxes, signal speeds and face speeds go
@@ -2801,7 +2803,7 @@ __global__ void __launch_bounds__(256) k_mlp_adam(const float* __restrict__ part
 // hidden values a thread would halve the occupancy of the other.  The MFMA
 // path is bound by the vector ALU (about 1200 instructions per 64 states: 64
 // first-layer units in the rounding order of the FP32 sum, the output layer,
-// three logarithms and an exponential in FP64): 2^20 states 77 -> 35 us.
+// three logarithms and an exponential in FP64): 2^20 states 77 -> 37 us.
 // The FP32 path packs nothing for a workgroup to share, so it takes one
 // wavefront a workgroup, which spreads small batches over the most CUs (64
 // against 256 threads: 1 to 3000 states 26.0-26.8 against 29.2-30.6 us, 10,000
