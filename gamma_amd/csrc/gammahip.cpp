@@ -2263,20 +2263,18 @@ __device__ void wg_merge(const Dev& d, int j, long long b, int i, int* s_left) {
   }
   __syncthreads();
 }
-// The decisions of active cells lo .. hi of track j (rgflag), the last one past
-// the shock threshold and the first and last flagged, taken into best, f and l
-// by the workgroup's threads.  A decision depends on the shock index only in
-// the nine cells past it, so the cells are read once and judged without that
-// window (wg_screen).
-template <int ND, int NQ>
-__device__ void wg_judge(const Dev& d, int j, bool bm, int lo, int hi, int& best, int& f, int& l) {
+// The decisions of active cells lo .. hi of track j by the workgroup's threads
+// (rgflag, and found(cell) for each flagged one), and the last cell past the
+// shock threshold.  A decision depends on the shock index only in the nine
+// cells past it, so the cells are read once and judged without that window
+// (wg_screen).
+template <int ND, int NQ, class Found>
+__device__ __forceinline__ void wg_judge(const Dev& d, int j, bool bm, int lo, int hi, int& best, const Found& found) {
   int nt = d.ntrack[j], iR = nt - d.ngst, t = (int)threadIdx.x;
   long long b = CI(d, j, 0);
   double thr = 1.5 * d.rg[3];
   auto flag = [&](int i, int a) {
-    if (!rg_flag(d, b, i, nt, a)) return;
-    f = f < i ? f : i;
-    l = i > l ? i : l;
+    if (rg_flag(d, b, i, nt, a)) found(i);
   };
   if (d.trg[j] == RG_USER) {
     for (int i = lo + t; i <= hi; i += RGB) flag(i, rg_check<ND, NQ>(d, j, i, HUGE_VAL));
@@ -2301,49 +2299,55 @@ __device__ void wg_judge(const Dev& d, int j, bool bm, int lo, int hi, int& best
     for (int u = 0; u < U; ++u) {
       int m = i + u * RGB;
       if (m > hi) break;
-      if (bm && pp[u] > thr && m > best) best = m;
+      if (bm && pp[u] > thr) best = m;          // m grows
       flag(m, bm ? rg_rule_bm(d, dx[u], lfac<ND, NQ>(p[u]), -HUGE_VAL, rOut) : rg_rule_ar(d, dx[u], dy));
     }
   }
 }
-// One pass over the workgroup's track ahead of the loop: body_rg_shockpos and
-// body_rg_screen.  The shock index is exact; i0 .. i1 hold every flagged cell,
-// but cells that only the window unflagged may lie at their ends (the loop
-// goes by rgflag, or judges the cells itself).
+// One pass over the workgroup's track ahead of the loop: every active cell's
+// decision, the shock index and the first and last flagged cell, all of
+// body_rg_shockpos and body_rg_screen.  CW: k_rg_screen's findings are taken
+// instead; then cells that only the window unflagged may lie at the ends of
+// i0 .. i1 (the loop goes by rgflag, or judges the cells itself).
 // One launch instead of four (clear, shock position, screen, loop): a regrid
 // without actions takes 8 instead of 17 us on one 4000-cell track, 39 instead
 // of 62 us on 256 tracks of 512-16384 cells, 30 us either way on 2048 x 2048.
-template <int ND, int NQ>
+template <int ND, int NQ, bool CW>
 __device__ bool wg_screen(const Dev& d, int j, bool bm, int* red, int* i0, int* i1, double* iS) {
   int nt = d.ntrack[j], iL = d.ngst - 1, iR = nt - d.ngst, t = (int)threadIdx.x;
-  int best = iL + 1, f = INT_MAX, l = -1;
-  if (d.rgch) {                         // k_rg_screen has judged the cells
+  long long b = CI(d, j, 0);
+  int best = iL + 1, any = 0, f = INT_MAX, l = -1;
+  if (CW) {
     for (int q = t; q < d.rgch; q += RGB) {
       const int* p = d.rgpart + 3 * ((long long)j * d.rgch + q);
-      best = p[0] > best ? p[0] : best;
-      f = p[1] < f ? p[1] : f;
-      l = p[2] > l ? p[2] : l;
+      best = max(best, p[0]);
+      f = min(f, p[1]);
+      l = max(l, p[2]);
     }
+    any = l >= 0;
   } else {
-    wg_judge<ND, NQ>(d, j, bm, iL + 1, iR - 1, best, f, l);
+    wg_judge<ND, NQ>(d, j, bm, iL + 1, iR - 1, best, [&](int) { any = 1; });
   }
   *iS = 0.;
   if (bm) {
     int s = wg_reduce<true>(best, red);
     *iS = (double)s;
     int m = s + 1 + t;
-    if (t < 9 && m <= iR - 1 && rg_flag(d, CI(d, j, 0), m, nt, rg_check<ND, NQ>(d, j, m, *iS))) {
-      f = m < f ? m : f;
-      l = m > l ? m : l;
+    if (t < 9 && m <= iR - 1 && rg_flag(d, b, m, nt, rg_check<ND, NQ>(d, j, m, *iS))) {
+      any = 1;
+      if (CW) { f = min(f, m); l = max(l, m); }
     }
   }
+  if (!wg_reduce<true>(any, red)) return false;
+  if (!CW)
+    for (int i = iL + 1 + t; i <= iR - 1; i += RGB)
+      if (d.rgflag[b + i]) { f = min(f, i); l = i; }
   *i0 = wg_reduce<false>(f, red);
-  if (*i0 == INT_MAX) return false;
   *i1 = wg_reduce<true>(l, red);
   __syncthreads();
-  return true;
+  return *i1 >= 0;
 }
-template <int ND, int NQ>
+template <int ND, int NQ, bool CW>
 __device__ void wg_regrid(const Dev& d, int j) {
   __shared__ int red[RGB];
   __shared__ double rv[RGB];
@@ -2353,7 +2357,7 @@ __device__ void wg_regrid(const Dev& d, int j) {
   long long b = CI(d, j, 0);
   int i, tl;
   double iS;
-  if (!wg_screen<ND, NQ>(d, j, bm, red, &i, &tl, &iS)) return;
+  if (!wg_screen<ND, NQ, CW>(d, j, bm, red, &i, &tl, &iS)) return;
   int is = -1, ib = -1;
   if (d.circ) wg_victims<ND, NQ>(d, j, rv, red, &is, &ib);
   RgStop stop = rg_stop_init(d, j, iS, tl);
@@ -2442,7 +2446,11 @@ __global__ void __launch_bounds__(RGB) k_rg_screen(Dev d, int reset) {
   if (!active_track(d, j) || d.trg[j] == RG_NONE) return;
   int iL = d.ngst - 1, iR = d.ntrack[j] - d.ngst, v[3] = {iL + 1, -INT_MAX, -1};   // best, -first, last
   int lo = max(s0, iL + 1), hi = min(s0 + d.rgspan, iR) - 1, f = INT_MAX;
-  if (lo <= hi) wg_judge<ND, NQ>(d, j, d.trg[j] == RG_BM1D, lo, hi, v[0], f, v[2]);
+  if (lo <= hi)
+    wg_judge<ND, NQ>(d, j, d.trg[j] == RG_BM1D, lo, hi, v[0], [&](int i) {
+      f = min(f, i);
+      v[2] = max(v[2], i);
+    });
   v[1] = -f;
   for (int o = 32; o > 0; o >>= 1)
     for (int q = 0; q < 3; ++q) v[q] = max(v[q], __shfl_xor(v[q], o, 64));
@@ -2454,20 +2462,20 @@ __global__ void __launch_bounds__(RGB) k_rg_screen(Dev d, int reset) {
   for (int w = 1; w < RGB / 64; ++w) m = max(m, red[w][t]);
   d.rgpart[3 * (long long)blockIdx.x + t] = t == 1 ? -m : m;
 }
-template <int ND, int NQ>
+template <int ND, int NQ, bool CW>
 __global__ void __launch_bounds__(RGB) k_regrid(Dev d, int reset) {
-  if (reset && !d.rgch)                 // no rule or action reads the shock state
+  if (reset && !CW)                     // no rule or action reads the shock state
     for (int i = (int)threadIdx.x; i < d.nax; i += RGB) body_shock_reset(d, (int)blockIdx.x, i);
-  wg_regrid<ND, NQ>(d, (int)blockIdx.x);
+  wg_regrid<ND, NQ, CW>(d, (int)blockIdx.x);
 }
 
 // ---- the five passes of a 1D step (see s1_face1) ----
 // begin: one workgroup per track; RG: some track has a regrid rule
-template <int NQ, bool RG>
+template <int NQ, bool RG, bool CW>
 __global__ void __launch_bounds__(RG ? RGB : 64) k1_begin(Dev d) {
   int j = (int)blockIdx.x;
   if (RG) {
-    wg_regrid<1, NQ>(d, j);
+    wg_regrid<1, NQ, CW>(d, j);
     __syncthreads();
   }
   if ((int)threadIdx.x < 2 * d.ngst) body_ghost_mv<1, NQ>(d, j, (int)threadIdx.x);
@@ -2512,8 +2520,8 @@ __global__ void __launch_bounds__(S1B) k1_faces(Dev d) {
     d.tpart[(long long)j * d.s1ch + blockIdx.x] = m;
   }
 }
-// the minimum of each track's tiles, ahead of the first stage, where there are
-// too many for every wavefront of the stage to read
+// the minimum of each track's tiles into the first of them, ahead of the first
+// stage, where there are too many for every wavefront of the stage to read
 __global__ void __launch_bounds__(1024) k1_dt_min(Dev d) {
   __shared__ double sm[16];
   int j = (int)blockIdx.x, t = (int)threadIdx.x, n = (d.ntrack[j] + S1C - 1) / S1C;
@@ -2524,7 +2532,7 @@ __global__ void __launch_bounds__(1024) k1_dt_min(Dev d) {
   __syncthreads();
   if (t) return;
   for (int q = 1; q < 16; ++q) m = fmin(m, sm[q]);
-  d.tmin[j] = m;
+  d.tpart[(long long)j * d.s1ch] = m;     // after the barrier: all tiles are read
 }
 template <int NQ, bool SHK, int SV, int STAGE, bool STD>
 __global__ void __launch_bounds__(S1B) k1_stage(Dev d) {
@@ -2537,18 +2545,13 @@ __global__ void __launch_bounds__(S1B) k1_stage(Dev d) {
   double dt;
   if (STAGE == 1) {
     // the track's minimum over its tiles, by every wavefront for itself (a
-    // minimum does not depend on the order it is taken in), or k1_dt_min's
+    // minimum does not depend on the order it is taken in); k1_dt_min leaves one
     double m = 1.e15;
-    int n = (nt + S1C - 1) / S1C;
-    if (d.s1min) m = d.tmin[j];
-    else for (int q = t & 63; q < n; q += 64) m = fmin(m, d.tpart[(long long)j * d.s1ch + q]);
-    if (!d.s1min)
-      for (int s = 32; s > 0; s >>= 1) m = fmin(m, __shfl_xor(m, s, 64));
+    int n = d.s1min ? 1 : (nt + S1C - 1) / S1C;
+    for (int q = t & 63; q < n; q += 64) m = fmin(m, d.tpart[(long long)j * d.s1ch + q]);
+    for (int s = 32; s > 0; s >>= 1) m = fmin(m, __shfl_xor(m, s, 64));
     dt = d.P.cfl * m;
-    if (blockIdx.x == 0 && t == 0) {
-      if (!d.s1min) d.tmin[j] = m;
-      d.tdt[j] = dt;
-    }
+    if (blockIdx.x == 0 && t == 0) { d.tmin[j] = m; d.tdt[j] = dt; }
   } else {
     dt = d.tdt[j];
   }
@@ -3512,7 +3515,8 @@ struct Pipe {
     if (reset) L2(c, body_shock_reset, d.nj, d.nax);
 #else
     rg_screen(c, reset);
-    hipLaunchKernelGGL((k_regrid<ND, NQ>), dim3(d.nj), dim3(RGB), 0, c->stream, d, reset ? 1 : 0);
+    if (d.rgch) hipLaunchKernelGGL((k_regrid<ND, NQ, true>), dim3(d.nj), dim3(RGB), 0, c->stream, d, reset ? 1 : 0);
+    else hipLaunchKernelGGL((k_regrid<ND, NQ, false>), dim3(d.nj), dim3(RGB), 0, c->stream, d, reset ? 1 : 0);
 #endif
   }
   static void apply(gammahip_ctx* c, int what) {
@@ -3585,9 +3589,13 @@ struct Pipe {
     };
 #else
     dim3 tiles(d.s1ch, d.nj);
-    if (d.rg_mode) rg_screen(c, false);
-    if (d.rg_mode) hipLaunchKernelGGL((k1_begin<NQ, true>), dim3(d.nj), dim3(RGB), 0, c->stream, d);
-    else hipLaunchKernelGGL((k1_begin<NQ, false>), dim3(d.nj), dim3(64), 0, c->stream, d);
+    if (!d.rg_mode) {
+      hipLaunchKernelGGL((k1_begin<NQ, false, false>), dim3(d.nj), dim3(64), 0, c->stream, d);
+    } else {
+      rg_screen(c, false);
+      if (d.rgch) hipLaunchKernelGGL((k1_begin<NQ, true, true>), dim3(d.nj), dim3(RGB), 0, c->stream, d);
+      else hipLaunchKernelGGL((k1_begin<NQ, true, false>), dim3(d.nj), dim3(RGB), 0, c->stream, d);
+    }
     bool std = !d.P.synge && !d.pc && !d.vpspec;
     tbeg(c, 1);
     if (std) hipLaunchKernelGGL((k1_faces<NQ, SHK, true>), tiles, dim3(S1B), 0, c->stream, d);
